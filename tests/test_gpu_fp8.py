@@ -27,6 +27,29 @@ def test_quantize_rows_bit_exact(dev):
     assert np.array_equal(q2.cpu().numpy(), oq2) and np.array_equal(s2.cpu().numpy(), os2)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("R,C", [(1, 8), (3, 72), (5, 2048), (600, 2056), (2, 16384), (3, 28672),
+                                 (2, 65544)])
+def test_quantize_rows_units(dev, dtype, R, C):
+    # rows of whole 16-byte units (the one-workgroup-per-row form: 1..8 units
+    # per thread, partly filled, and longer than it takes) against the oracle:
+    # zeros of both signs, infinities, NaN, midpoints between two codes, scales
+    # where the row divides
+    g = torch.Generator().manual_seed(R + C)
+    x = torch.randn(R, C, generator=g) * torch.exp(2 * torch.randn(R, 1, generator=g))
+    x[0, :8] = torch.tensor([0.0, -0.0, 17.0, -19.0, 2.0**-10, 3 * 2.0**-10, 448.0, -232.0])
+    if R > 1:
+        x[1] *= 1e-30
+        x[R - 1, C - 1] = float("inf")
+    x = x.to(dtype)
+    q, s = fp8.quantize_rows(x.to(dev))
+    want_q, want_s = oracle.fp8_quantize_rows(x.float().numpy())
+    q, s = q.cpu().numpy(), s.cpu().numpy()
+    assert np.array_equal(s, want_s)
+    nan = (want_q & 0x7F) == 0x7F  # inf / inf: NaN, its sign is not fixed
+    assert np.array_equal(q[~nan], want_q[~nan]) and np.all((q[nan] & 0x7F) == 0x7F)
+
+
 def test_prepack_transpose(dev):
     w = torch.randint(0, 256, (200, 72), dtype=torch.uint8, device=dev)
     assert torch.equal(fp8.prepack_weight(w), w.T.contiguous())
