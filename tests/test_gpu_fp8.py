@@ -85,6 +85,26 @@ def test_fp8_gemm_vs_oracle(dev, fp8_variant, M, K, N):
     assert rel_err(got, a.double().numpy() @ w.double().numpy()) < 8e-2
 
 
+@pytest.mark.parametrize("K,N", [(128, 8), (384, 40), (1024, 16400), (1152, 520), (1920, 8200),
+                                 (2176, 4099), (4096, 16400), (4224, 300), (8192, 4136)])
+@pytest.mark.parametrize("M", [1, 7, 16])
+def test_fp8_decode(dev, M, K, N):
+    # up to 16 tokens: every step count / tile width of the decode kernel, K
+    # with idle wavefronts, ragged N, more than one tile per workgroup
+    g = torch.Generator(device=dev).manual_seed(M + K + N)
+    aq, sa = fp8.quantize_rows(torch.randn(M, K, device=dev, generator=g))
+    wq, sw = fp8.quantize_rows(torch.randn(N, K, device=dev, generator=g))
+    guard = torch.full((M + 1, N), 3.0, device=dev, dtype=torch.bfloat16)
+    out = fp8.gemm(aq, sa, wq, sw, out=guard[:M])
+    dec = lambda q: q.view(torch.float8_e4m3fn).double()
+    want = (dec(aq) * sa.double()[:, None]) @ (dec(wq) * sw.double()[:, None]).T.contiguous()
+    # every output: one bf16 rounding (2^-9) of a sum whose f32 error is far below it
+    err = (out.double() - want).abs()
+    rms = want.square().mean().sqrt()
+    assert bool((err <= 2.0**-8 * want.abs() + 1e-4 * rms).all()), (err / rms).max()
+    assert bool((guard[M] == 3.0).all())
+
+
 @pytest.mark.parametrize("M", [256, 4096])
 def test_fp8_cfg5(dev, fp8_variant, M):
     # configs[4] shapes K=8192, N=28672; M = 4096 is the full config (16 row

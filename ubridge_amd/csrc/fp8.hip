@@ -313,6 +313,133 @@ k_fp8_gemm2(const uint8_t* __restrict__ A, const float* __restrict__ sa,
     }
 }
 
+// Decode batches (at most 16 tokens): the product is a stream of the weight,
+// HBM-bound, so the kernel is shaped for bytes in flight.  A persistent grid
+// of W-wavefront workgroups walks tiles of 16 RT weight rows.  The W
+// wavefronts split K (wavefront w the 128-byte steps w, w + W, ...: at most
+// SP), so a wavefront's activation fragments are the same for every tile
+// and stay in SP registers sets for the whole launch; per tile it holds SP x
+// RT weight fragments, straight from memory, and the next tile's loads are in
+// flight while the current one is multiplied and summed (two register sets,
+// the tile loop unrolled by two).  A fragment is two 16-byte loads per lane,
+// lane (r, h) reading bytes 16 h and 64 + 16 h of row r's 128, so a load
+// covers 64-byte runs of 16 rows (the k order inside the step is the same on
+// both operands, which leaves the dot unchanged).
+// v_mfma_scale_f32_16x16x128_f8f6f4 (block scales 2^0), tokens as A rows:
+// lane (r, h) ends with tokens 4 h .. 4 h + 3 of weight row r.  The partial
+// sums meet in LDS in wavefront order, in one of two buffers by tile parity,
+// so one barrier per tile suffices.
+template <int W, int SP, int RT>
+__global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4, 4)))
+k_fp8_dec(const uint8_t* __restrict__ A, const float* __restrict__ sa,
+          const uint8_t* __restrict__ Wt, const float* __restrict__ sw,
+          uint16_t* __restrict__ out, int M, int K, int N) {
+  typedef float f32x4 __attribute__((ext_vector_type(4)));
+  constexpr int NR = 16 * RT, NRP = NR + 1;  // padded row of partial sums
+  __shared__ float red[2][W * 16 * NRP];
+  const int tid = threadIdx.x, lane = tid & 63, r = lane & 15, h = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const __amdgpu_buffer_rsrc_t ra = rsrc(A, (uint64_t)M * K);
+  const __amdgpu_buffer_rsrc_t rw = rsrc(Wt, (uint64_t)N * K);
+  const int steps = K / 128, nt = (N + NR - 1) / NR, G = gridDim.x;
+  const uint32_t lo = (uint32_t)r * (uint32_t)K + 16u * (uint32_t)h;
+  uint32_t ko[SP];  // byte offset of the wavefront's step i, kOOB past K
+#pragma unroll
+  for (int i = 0; i < SP; i++) ko[i] = wave + i * W < steps ? (uint32_t)(wave + i * W) * 128u : kOOB;
+  auto frag = [](const uint4 (&v)[2]) -> i32x8 {
+    return (i32x8){(int)v[0].x, (int)v[0].y, (int)v[0].z, (int)v[0].w,
+                   (int)v[1].x, (int)v[1].y, (int)v[1].z, (int)v[1].w};
+  };
+  // rows >= N (and tiles >= nt) lie past the end of the buffer: zero
+  auto load = [&](uint4 (&b)[SP][RT][2], int t) {
+    const uint32_t base = lo + (uint32_t)t * (uint32_t)(NR * K);
+#pragma unroll
+    for (int i = 0; i < SP; i++)
+#pragma unroll
+      for (int j = 0; j < RT; j++)
+#pragma unroll
+        for (int q = 0; q < 2; q++)
+          b[i][j][q] = ld16(rw, ko[i] == kOOB ? kOOB : base + (uint32_t)(16 * j * K) + ko[i] + 64u * q);
+  };
+  uint4 a[SP][2], b0[SP][RT][2], b1[SP][RT][2];
+  load(b0, blockIdx.x);
+#pragma unroll
+  for (int i = 0; i < SP; i++)
+#pragma unroll
+    for (int q = 0; q < 2; q++) a[i][q] = ld16(ra, ko[i] == kOOB ? kOOB : lo + ko[i] + 64u * q);
+  const float sat = tid < 16 * NR && tid / NR < M ? sa[tid / NR] : 0.f;
+  auto tile = [&](const uint4 (&b)[SP][RT][2], int t, int p) {
+    f32x4 acc[RT];
+#pragma unroll
+    for (int j = 0; j < RT; j++) acc[j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < SP; i++)
+#pragma unroll
+      for (int j = 0; j < RT; j++)
+        acc[j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(frag(a[i]), frag(b[i][j]), acc[j],
+                                                                  0, 0, 0, 127, 0, 127);
+#pragma unroll
+    for (int j = 0; j < RT; j++)
+#pragma unroll
+      for (int i = 0; i < 4; i++) red[p][(wave * 16 + 4 * h + i) * NRP + 16 * j + r] = acc[j][i];
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the partial sums are written
+    ub_barrier();                        // (the next tile's loads stay in flight)
+    if (tid < 16 * NR) {  // 16 NR <= 64 W
+      const int m = tid / NR, n = t * NR + tid % NR;
+      float v = 0.f;
+#pragma unroll
+      for (int w = 0; w < W; w++) v += red[p][(w * 16 + m) * NRP + tid % NR];
+      if (m < M && n < N)
+        out[(size_t)m * N + n] = __builtin_bit_cast(unsigned short, (__bf16)(v * sat * sw[n]));
+    }
+  };
+  for (int t = blockIdx.x; t < nt; t += 2 * G) {
+    load(b1, t + G);
+    tile(b0, t, 0);
+    if (t + G >= nt) break;  // uniform
+    load(b0, t + 2 * G);
+    tile(b1, t + G, 1);
+  }
+}
+
+// The decode kernel takes up to 16 tokens, K a multiple of 128 up to 8192
+// (four steps of 16 wavefronts; longer rows would not leave registers for the
+// activations) and 32-bit weight offsets.  Against hipBLASLt's fp8 GEMM, us at
+// 1 / 16 tokens, weights rotated over 600 MB (hipBLASLt -> this kernel):
+// 8192 x 28672 58 / 57 -> 42 / 44 (5.3 TB/s at 16), 5120 x 17408 36 / 36 -> 21
+// / 22, 4096 x 14336 26 / 16 -> 12.8 / 13.7, 4096 x 4096 12 / 12 -> 5.7 / 6.8,
+// 8192 x 8192 42 / 16 -> 14 / 16, 1024 x 8192 9.6 / 7.9 -> 4.0 / 4.6.  From 17
+// tokens hipBLASLt is as fast (8192 x 28672 48 at 20 tokens against 57 for two
+// activation tiles here).  RT: wider tiles where a wavefront has few steps,
+// so that 4 fragments are in flight per register set, as long as the tiles
+// still cover the CUs.
+bool fp8_dec(const uint8_t* a, const float* sa, const uint8_t* w, const float* sw, uint16_t* out,
+             int M, int K, int N, hipStream_t s) {
+  if (M > 16 || K < 128 || K % 128 != 0 || K > 8192 || (uint64_t)N * K >= 0x80000000ull ||
+      (((uintptr_t)a | (uintptr_t)w) & 15) != 0)
+    return false;
+  const int steps = K / 128;
+#define UB_DEC(W_, SP_, RT_)                                                             \
+  {                                                                                      \
+    const int nt = ub_cdiv(N, 16 * RT_), cap = 256 * 16 / W_;                            \
+    k_fp8_dec<W_, SP_, RT_><<<nt < cap ? nt : cap, 64 * W_, 0, s>>>(a, sa, w, sw, out, M, K, N); \
+    return true;                                                                         \
+  }
+  if (steps > 32) UB_DEC(16, 4, 1)
+  if (steps > 16) {
+    if (N >= 16384) UB_DEC(16, 2, 2)
+    UB_DEC(16, 2, 1)
+  }
+  if (steps > 8) {
+    if (N >= 16384) UB_DEC(16, 1, 4)
+    if (N >= 8192) UB_DEC(16, 1, 2)
+    UB_DEC(16, 1, 1)
+  }
+  if (N >= 16384) UB_DEC(8, 1, 2)
+  UB_DEC(8, 1, 1)
+#undef UB_DEC
+}
+
 // [R, C] bytes -> [C, R] bytes through a 64 x 64 LDS tile.
 __global__ void __launch_bounds__(256) k_transpose_u8(const uint8_t* __restrict__ in,
                                                       uint8_t* __restrict__ out, int R, int C) {
@@ -473,14 +600,17 @@ UB_API int ubridge_fp8_gemm(const uint8_t* a, const float* sa, const uint8_t* w_
   dim3 grid(ub_cdiv(N, FBN) * ub_cdiv(M, FBM));
   const int tile = ub_tune(UB_TUNE_GEMM_TILE);
   hipStream_t s = ub_stream(stream);
-  // By default hipBLASLt's fp8 GEMM with per-row / per-column scale vectors
-  // (configs[4] on MI355X: 753-757 against 882-888 us for the kernels below),
-  // falling back to them when the library cannot serve the shape.  Knob
-  // gemm_tile 3: the 128-byte K-step kernel below (one barrier per 16
+  // Up to 16 tokens k_fp8_dec (fp8_dec has the figures); beyond, hipBLASLt's
+  // fp8 GEMM with per-row / per-column scale vectors (4096 x 8192 x 28672:
+  // 753-757 against 882-888 us for the kernels below), falling back to them
+  // when the library cannot serve the shape.  Knob gemm_tile 1: hipBLASLt at
+  // every size, 3: the 128-byte K-step kernel below (one barrier per 16
   // MFMAs when K allows: 912 -> 883 us), 2: the 4-wavefront kernel, 4: the
   // 8-wavefront one with 64-byte K-steps.
   if (tile == 0 || tile == 1) {
     ub_blaslt_prepare(s);
+    if (tile == 0 && fp8_dec(a, sa, w_nk, sw, (uint16_t*)out, M, K, N, s))
+      return ub_check_launch(nm);
     const int e = ub_blaslt_fp8(a, sa, w_nk, sw, out, M, K, N, s);
     if (e != UB_ERR_UNSUPPORTED) return e ? e : ub_check_launch(nm);
   }
