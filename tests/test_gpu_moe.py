@@ -6,7 +6,7 @@ import torch
 
 import oracle
 from conftest import rel_err
-from ubridge_amd import moe, ops, synth
+from ubridge_amd import _lib, moe, ops, synth
 
 pytestmark = pytest.mark.gpu
 
@@ -163,6 +163,102 @@ def test_fused_moe_multi_step(dev, K, N, bs, q8, mrw, dtype):
     got = C.double().cpu()
     assert (got[em < 0] == 0).all()
     assert rel_err(got.numpy(), want.numpy()) < 1e-2
+
+
+@pytest.fixture
+def moe_path():
+    yield lambda v: ops.tune_set("moe_gemm_path", v)
+    ops.tune_set("moe_gemm_path", 0)
+
+
+@pytest.mark.parametrize("K,N,bs,q8,mrw,bias,emap,dtype", [
+    (64, 8, 32, True, 0, False, False, torch.bfloat16),      # one K-step, one column block's edge
+    (128, 264, 32, True, 1, True, True, torch.bfloat16),     # partial column block, -1 and shared experts
+    (192, 520, 16, False, 1, False, True, torch.bfloat16),
+    (320, 256, 64, False, 0, True, False, torch.float16),
+    (64, 48, 128, True, 1, False, False, torch.float16),
+    (448, 72, 1, False, 0, False, True, torch.bfloat16)])
+def test_moe_tile_kernel(dev, moe_path, K, N, bs, q8, mrw, bias, emap, dtype):
+    # 128-row tiles: experts with 0, 1, 31 .. 33, 95 .. 97, 127 .. 129, 300
+    # rows, against f64, rows of experts mapped to -1 zeroed, everything past
+    # the slots untouched
+    rows = [0, 1, 31, 32, 33, 0, 64, 65, 95, 96, 97, 127, 128, 129, 300, 2]
+    E, k = len(rows), 2
+    g = torch.Generator().manual_seed(K + N)
+    flat = torch.cat([torch.full((n,), e) for e, n in enumerate(rows)])
+    flat = flat[torch.randperm(flat.numel(), generator=g)]
+    T = flat.numel() // k
+    ids = flat[:T * k].view(T, k).int().to(dev)
+    em = None
+    if emap:  # neighbours 2 and 3 share an expert's weights, 6 and 14 are elsewhere
+        em = torch.arange(E, dtype=torch.int32)
+        em[3], em[6], em[14] = 2, -1, -1
+        em = em.to(dev)
+    s, e, n = moe.moe_align_block_size(ids, E, bs, expert_map=em)
+    A = torch.randn(T * k if mrw else T, K, generator=g).to(dtype).to(dev)
+    if q8:
+        B = torch.randint(-128, 128, (E, N, K), generator=g, dtype=torch.int8).to(dev)
+        Bs = (torch.rand(E, N, generator=g) * 0.01 + 0.001).to(dtype).to(dev)
+        Bf = B.double() * Bs.double()[:, :, None]
+    else:
+        B, Bs = torch.randn(E, N, K, generator=g).to(dtype).to(dev), None
+        Bf = B.double()
+    bv = torch.randn(E, N, generator=g).to(dtype).to(dev) if bias else None
+    tw = torch.rand(T * k, generator=g).to(dev)
+    C = torch.full((T * k + 1, N), 3.0, dtype=dtype, device=dev)
+    moe_path(10)
+    moe.invoke_fused_moe(A, B, C[:T * k], tw if mrw else None, s, e, n, k, bs, mrw, B_scale=Bs,
+                         bias=bv)
+    ex = ids.flatten().long() if em is None else em.long()[ids.flatten().long()]
+    here = ex >= 0
+    a = A.double() if mrw else A.double().repeat_interleave(k, 0)
+    want = torch.zeros(T * k, N, dtype=torch.float64, device=dev)
+    for q in range(E):
+        r = ex == q
+        want[r] = a[r] @ Bf[q].T.contiguous() + (bv[q].double() if bias else 0.0)
+    if mrw:
+        want *= tw.double()[:, None] * here[:, None]
+    got = C[:T * k].double()
+    assert bool((got[~here] == 0).all()) and bool((C[T * k] == 3.0).all())
+    # one rounding to T of an f32 sum (error far below it)
+    ulp = 2.0**-8 if dtype == torch.bfloat16 else 2.0**-10
+    rms = want[here].square().mean().sqrt()
+    assert bool(((got - want).abs() <= ulp * want.abs() + 1e-4 * rms).all())
+
+
+def test_moe_tile_windows(dev, moe_path):
+    # more tiles than the list in LDS holds (512): 700 experts of one block
+    # and 5 large ones; the same bits as the 32-row kernel
+    E, k, K, N = 705, 1, 64, 40
+    g = torch.Generator().manual_seed(1)
+    flat = torch.cat([torch.arange(700)] + [torch.full((200,), 700 + i) for i in range(5)])
+    ids = flat[torch.randperm(flat.numel(), generator=g)].int().view(-1, 1).to(dev)
+    s, e, n = moe.moe_align_block_size(ids, E, 32)
+    A = torch.randn(ids.shape[0], K, generator=g).bfloat16().to(dev)
+    B = torch.randn(E, N, K, generator=g).bfloat16().to(dev)
+    out = []
+    for path in (1, 10):
+        moe_path(path)
+        C = torch.zeros(ids.shape[0], N, dtype=torch.bfloat16, device=dev)
+        out.append(moe.invoke_fused_moe(A, B, C, None, s, e, n, k, 32, False))
+    assert torch.equal(out[0].view(torch.int16), out[1].view(torch.int16))
+
+
+def test_moe_tile_bad_expert_flagged(dev, moe_path):
+    # an expert id past E in experts_ids: its rows are left alone and the
+    # device flag is set
+    ids = torch.arange(4, dtype=torch.int32, device=dev).repeat(16, 1)
+    s, e, n = moe.moe_align_block_size(ids, 4, 16)
+    e[3] = 9
+    A = torch.randn(16, 64, device=dev).bfloat16()
+    B = torch.randn(4, 16, 64, device=dev).bfloat16()
+    C = torch.full((64, 16), 3.0, dtype=torch.bfloat16, device=dev)
+    moe_path(10)
+    moe.invoke_fused_moe(A, B, C, None, s, e, n, 4, 16, False)
+    with pytest.raises(_lib.UbridgeError):
+        moe.device_error()
+    assert bool((C[ids.flatten() == 3] == 3.0).all())
+    assert not bool((C[ids.flatten() < 3] == 3.0).all(1).any())
 
 
 def test_fused_moe_expert_minus_one_zeroes(dev):

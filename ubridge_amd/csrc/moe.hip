@@ -2,7 +2,8 @@
 //
 //   topk_softmax_{f32,f16,bf16}   topk_softmax_host.cpp:103-208
 //   moe_align_block_size          moe_align_host.cpp:51-935
-//   invoke_fused_moe_{bf16,f16}   fused_moe_host.cpp:43-536  (+ W8A16 variant)
+//   invoke_fused_moe_{bf16,f16}   fused_moe_host.cpp:43-536  (+ W8A16 variant;
+//                                 experts with many rows: moe_tile.hip)
 //   silu_and_mul / moe_sum        the steps either side of the grouped GEMM
 //   moe_{f16,bf16}, indexed_moe_{f16,bf16}   moe_host.cpp:27-293 (legacy)
 //
@@ -12,9 +13,11 @@
 // ubridge_device_error() reads after synchronizing the stream.
 #include "common.h"
 #include "lds_dma.h"
+#include "moe.h"
 #include "registry.h"
 
 #include <algorithm>
+#include <atomic>
 
 namespace {
 
@@ -522,21 +525,6 @@ void align_small_launch(const int* ids, int* sorted, int* experts, int* ntpp, in
 // units against bank conflicts.
 constexpr int MBM = 32;  // rows of a sorted block per workgroup
 
-struct MoeArgs {
-  void* C;
-  const void* A;
-  const void* B;
-  const void* Bs;   // int8 path: per-channel scales T [E, N]
-  const void* bias; // T [E, N] or null
-  const float* tw;  // [topk_ids_size] or null
-  const int* sorted;
-  const int* eids;
-  const int* ntpp;
-  int K, N, E, tis, top_k, bs, mrw;
-  int act;  // 1: gated SiLU output C[s, n] = T(silu(g) u), g / u = weight rows n / N/2 + n
-  int a_div;  // slot s reads A row s / a_div
-};
-
 template <int DT>
 __device__ __forceinline__ f32x16 mfma(const uint4& a, const uint4& b, const f32x16& c) {
   if constexpr (DT == UB_BF16)
@@ -843,7 +831,8 @@ __global__ void __launch_bounds__(64 * NWV) k_moe_gemm(MoeArgs a) {
 // 2: 256 columns, BK 64, 4 stages; 3: 128 columns, BK 64, 6 stages;
 // 4: 256 columns, BK 128, 3 stages (int8 only); 5: 128 columns, BK 64,
 // 4 stages; 6 / 7: 64 columns, BK 64, 4 / 6 stages; 8: 128 columns, BK 64,
-// 3 stages; 9: 64 columns, BK 128, 3 stages.  Automatic (0): 1 for int8
+// 3 stages; 9: 64 columns, BK 128, 3 stages; 10: the 128-row tiles of
+// moe_tile.hip.  Automatic (0): 10 where ub_moe_tile_pays, else 1 for int8
 // experts with K >= 1536 and for 16-bit experts, else 8 -- measured on
 // MI355X at the Qwen3-MoE shapes (gate/up K = 2048, down K = 768), where
 // both stream within ~2% of the same ring with the MFMA work removed.
@@ -874,6 +863,24 @@ void moe_gemm_launch(int path, const MoeArgs& a, int max_blocks, hipStream_t s) 
   }
 }
 
+// Address of g_device_error on the current device (null: not available).
+int* error_flag() {
+  static std::atomic<int*> cache[64];
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return nullptr;
+  int* p = cache[dev].load(std::memory_order_acquire);
+  if (!p) {
+    void* q = nullptr;
+    if (hipGetSymbolAddress(&q, HIP_SYMBOL(g_device_error)) != hipSuccess) {
+      (void)hipGetLastError();
+      return nullptr;
+    }
+    p = (int*)q;
+    cache[dev].store(p, std::memory_order_release);
+  }
+  return p;
+}
+
 int moe_gemm(const char* nm, int dt, bool q8, void* C, const void* A, const void* B,
              const void* Bscale, const void* bias, const float* tw, const int* sorted,
              const int* eids, const int* ntpp, int M, int K, int N, int E, int tis, int top_k,
@@ -898,6 +905,9 @@ int moe_gemm(const char* nm, int dt, bool q8, void* C, const void* A, const void
   const int max_blocks = (tis + E * (bs - 1)) / bs;
   hipStream_t s = ub_stream(stream);
   const int path = ub_tune(UB_TUNE_MOE_GEMM_PATH);
+  if ((path == 10 || (path == 0 && ub_moe_tile_pays(a, q8))) &&
+      ub_moe_tile(a, dt, q8, error_flag(), s))
+    return ub_check_launch(nm);
   if (dt == UB_BF16) {
     if (q8) moe_gemm_launch<UB_BF16, true>(path, a, max_blocks, s);
     else moe_gemm_launch<UB_BF16, false>(path, a, max_blocks, s);
