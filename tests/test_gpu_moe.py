@@ -44,7 +44,9 @@ def test_topk_softmax_ties(dev):
 @pytest.mark.parametrize("T,k,E,bs", [(256, 8, 128, 16), (256, 8, 128, 64), (7, 2, 5, 4),
                                       (1, 1, 3, 8), (600, 4, 256, 32), (64, 8, 1024, 16),
                                       (4096, 8, 128, 32), (3000, 6, 60, 16), (5000, 2, 1024, 8),
-                                      (1000, 8, 7, 64), (700, 8, 128, 1)])
+                                      (1000, 8, 7, 64), (700, 8, 128, 1), (128, 8, 128, 32),
+                                      (129, 8, 128, 32), (1025, 1, 3, 32), (2048, 1, 1, 32),
+                                      (300001, 1, 60, 16), (270000, 4, 33, 1)])
 def test_moe_align_exact(dev, T, k, E, bs):
     ids = np.random.default_rng(T * E + bs).integers(0, E, (T, k)).astype(np.int32)
     s, e, n = moe.moe_align_block_size(torch.from_numpy(ids).to(dev), E, bs)
@@ -79,6 +81,21 @@ def test_moe_align_expert_map_real_tokens_large(dev):
         os_, oe, on = oracle.moe_align_block_size(ids, E, bs, real_token_num=rtn, expert_map=emap)
         assert n.item() == on[0]
         assert np.array_equal(s.cpu().numpy(), os_) and np.array_equal(e.cpu().numpy(), oe)
+
+
+@pytest.mark.parametrize("rt", [0, 1, 700, 5000])
+def test_moe_align_many_groups_map_tokens(dev, rt):
+    # several workgroups, ids that are not 16-byte aligned, part of the tokens
+    T, k, E, bs = 5000, 3, 40, 32
+    ids = np.random.default_rng(rt).integers(0, E, (T, k)).astype(np.int32)
+    emap = np.where(np.arange(E) % 4 == 1, -1, np.arange(E) // 2).astype(np.int32)
+    buf = torch.empty(T * k + 1, dtype=torch.int32, device=dev)
+    buf[1:] = torch.from_numpy(ids.ravel()).to(dev)
+    s, e, n = moe.moe_align_block_size(buf[1:].view(T, k), E, bs, real_token_num=rt,
+                                       expert_map=torch.from_numpy(emap).to(dev))
+    os_, oe, on = oracle.moe_align_block_size(ids, E, bs, real_token_num=rt, expert_map=emap)
+    assert n.item() == on[0]
+    assert np.array_equal(s.cpu().numpy(), os_) and np.array_equal(e.cpu().numpy(), oe)
 
 
 def test_moe_align_bad_ids_flagged(dev):

@@ -214,18 +214,24 @@ int topk_softmax_launch(const void* in, void* out, int* idx, int T, int E, int k
 }
 
 // ============================================================ moe_align_block_size
-// One workgroup of 1024 threads (16 wavefronts) for any slot count.  The
-// slots i = t*k + j are cut into chunks of 64 (one wavefront-wide load);
-// wavefront w takes a contiguous run of chunks.  Within a chunk the lanes
-// holding the same expert are found by one ballot per bit of the expert id,
-// so a slot's rank among equal experts earlier in the chunk is a popcount.
-// Pass 1 counts each wavefront's slots per expert (LDS row per wavefront,
-// updated by the first lane of each expert group; no atomics); the counts
-// are prefixed over wavefronts per expert and the padded expert offsets
-// scanned; pass 2 walks the same chunks again and places slot i at
-// eoff[e] + (slots of e in earlier wavefronts and chunks) + rank.  Slots of
-// one expert therefore keep ascending order, as the reference's stable
-// scatter (moe_align_host.cpp:766-921).
+// Any slot count, expert_map and real_token_num.  The slots i = t*k + j are
+// cut into runs, one per workgroup of 1024 threads (16 wavefronts).  Each
+// workgroup counts all the ids itself (LDS integer atomics; one histogram for
+// the slots before its run, one for the rest), so it knows every expert's
+// padded offset and where its own run starts inside each expert without a
+// second launch, scratch memory or a handoff between workgroups; then it
+// places its run 1024 slots at a time, one wavefront-wide chunk of 64 per
+// wavefront.  Within a chunk the lanes holding the same expert are found by
+// one ballot per bit of the expert id, so a slot's rank among equal experts is
+// a popcount; the chunks' counts meet in LDS.  Slots of one expert keep
+// ascending order, as the reference's stable scatter
+// (moe_align_host.cpp:766-921).  Padding, the tail and experts_ids are shared
+// out over the workgroups.
+// Latency-bound (counting 32,768 ids takes a workgroup ~32 LDS atomics per
+// thread).  One workgroup doing all of it is bound by its CU's scattered
+// stores and an LDS read-modify-write chain per wavefront: 128 experts, 4,096
+// / 8,192 / 32,768 / 131,072 slots 9.3 / 13.0 / 42.8 / 160 us, this way 6.2 /
+// 6.7 / 9.0 / 18.1.
 constexpr int kAlignThreads = 1024, kAlignWaves = kAlignThreads / 64;
 
 // lanes of this wavefront holding the same (non-negative) expert e
@@ -239,130 +245,129 @@ __device__ __forceinline__ uint64_t same_expert(int e, int nbits) {
   return m;
 }
 
+// LDS: before[E], rest[E], eoff[E + 1], cnt[kAlignWaves][E] (16 bits)
+size_t align_lds(int E) { return sizeof(int) * (3 * (size_t)E + 1) + 2 * (size_t)kAlignWaves * E; }
+
 __global__ void __launch_bounds__(kAlignThreads) k_moe_align(
     int* __restrict__ sorted, int* __restrict__ experts, int* __restrict__ ntpp,
     const int* __restrict__ ids, const int* __restrict__ real_tn, const int* __restrict__ emap,
-    int E, int bs, int T, int k) {
+    int E, int bs, int T, int k, int run) {
   extern __shared__ int sh[];
-  int* wcnt = sh;                    // [kAlignWaves][E]
-  int* eoff = wcnt + kAlignWaves * E;  // [E + 1]
-  __shared__ int bad;
+  int* before = sh;
+  int* rest = before + E;
+  int* eoff = rest + E;
+  uint16_t* cnt = (uint16_t*)(eoff + E + 1);
+  __shared__ int bad, wsum[kAlignWaves];
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const int g = blockIdx.x, G = gridDim.x;
   const int pad = T * k;
   const int max_padded = T * k + E * (bs - 1);
   const int max_blocks = max_padded / bs;
   const int nbits = E > 1 ? 32 - __clz(E - 1) : 0;
+  int tn = real_tn ? *real_tn : T;
+  bool any_bad = tn < 0 || tn > T;
+  if (any_bad) tn = 0;
+  const int n = tn * k, s0 = min(n, g * run), s1 = min(n, s0 + run);
   if (tid == 0) bad = 0;
-  for (int i = tid; i < kAlignWaves * E; i += kAlignThreads) wcnt[i] = 0;
-  __syncthreads();
-  int tn = T;
-  if (real_tn) {
-    tn = *real_tn;
-    if (tn < 0 || tn > T) { if (tid == 0) bad = 1; tn = 0; }
-  }
-  const int n = tn * k;
+  for (int i = tid; i < 2 * E; i += kAlignThreads) sh[i] = 0;
+  for (int i = tid; i < kAlignWaves * E; i += kAlignThreads) cnt[i] = 0;
   if (emap)
-    for (int e = tid; e < E; e += kAlignThreads)
-      if (emap[e] < -1 || emap[e] >= E) bad = 1;
-  // pad fill of both outputs (memsets at moe_align_host.cpp:777-784)
-  for (int i = tid; i < max_padded; i += kAlignThreads) sorted[i] = pad;
-  for (int i = tid; i < max_blocks; i += kAlignThreads) experts[i] = 0;
-  const int nc = (n + 63) / 64, cpw = (nc + kAlignWaves - 1) / kAlignWaves;
-  const int c0 = wv * cpw, c1 = min(nc, c0 + cpw);
-  int* mine = wcnt + wv * E;
-  const uint64_t below = (1ull << lane) - 1;
-  // the wavefront's ids, KB chunks at a time (independent loads in flight)
-  constexpr int KB = 8;
-  auto load_ids = [&](int cb, int (&ev)[KB]) {
-#pragma unroll
-    for (int q = 0; q < KB; q++) {
-      const int i = (cb + q) * 64 + lane;
-      ev[q] = cb + q < c1 && i < n ? ids[i] : -1;
-    }
+    for (int e = tid; e < E; e += kAlignThreads) any_bad |= emap[e] < -1 || emap[e] >= E;
+  __syncthreads();
+  auto count = [&](int e, int i) {
+    if ((unsigned)e >= (unsigned)E) any_bad = true;
+    else atomicAdd(i < s0 ? before + e : rest + e, 1);
   };
-  // pass 1: this wavefront's count per expert (and the id check)
-  bool any_bad = false;
-  for (int cb = c0; cb < c1; cb += KB) {
-    int ev[KB];
-    load_ids(cb, ev);
+  if (((uintptr_t)ids & 15) == 0) {  // four ids per load, four loads in flight
+    constexpr int U = 4;
+    for (int i0 = 4 * tid; i0 < n; i0 += 4 * U * kAlignThreads) {
+      int4 v[U];
 #pragma unroll
-    for (int q = 0; q < KB; q++) {
-      if (cb + q >= c1) break;
-      const int i = (cb + q) * 64 + lane;
-      any_bad |= i < n && (ev[q] < 0 || ev[q] >= E);
-      const int e = ev[q] >= 0 && ev[q] < E ? ev[q] : -1;
-      const uint64_t m = same_expert(e, nbits);
-      if (e >= 0 && __popcll(m & below) == 0) mine[e] += __popcll(m);
+      for (int u = 0; u < U; u++) {
+        const int i = i0 + 4 * u * kAlignThreads;
+        if (i + 3 < n) v[u] = *(const int4*)(ids + i);
+      }
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        const int i = i0 + 4 * u * kAlignThreads;
+        if (i + 3 < n) count(v[u].x, i), count(v[u].y, i + 1), count(v[u].z, i + 2), count(v[u].w, i + 3);
+        else for (int j = i; j < n; j++) count(ids[j], j);
+      }
     }
+  } else {
+    for (int i = tid; i < n; i += kAlignThreads) count(ids[i], i);
   }
   if (any_bad) bad = 1;
   __syncthreads();
-  if (bad) {
-    if (tid == 0) {
-      ntpp[0] = 0;
-      g_device_error = UB_ERR_INDEX;
+  const bool none = bad;  // a bad id, map entry or token count: no work
+  // padded offsets: an inclusive scan over the experts (E <= 1024: one each)
+  {
+    const int c = tid < E && !none ? before[tid] + rest[tid] : 0;
+    int v = (c + bs - 1) / bs * bs;
+    for (int o = 1; o < 64; o <<= 1) {
+      const int u = __shfl_up(v, o, 64);
+      if (lane >= o) v += u;
     }
-    return;
-  }
-  // exclusive prefix over wavefronts per expert; padded totals
-  for (int e = tid; e < E; e += kAlignThreads) {
-    int run = 0;
-    for (int w = 0; w < kAlignWaves; w++) {
-      const int v = wcnt[w * E + e];
-      wcnt[w * E + e] = run;
-      run += v;
-    }
-    eoff[e + 1] = (run + bs - 1) / bs * bs;
-  }
-  __syncthreads();
-  if (tid < 64) {  // inclusive scan of the padded counts, 64 at a time
-    int carry = 0;
-    for (int e0 = 0; e0 < E; e0 += 64) {
-      const int e = e0 + tid;
-      int v = e < E ? eoff[e + 1] : 0;
-      for (int o = 1; o < 64; o <<= 1) {
-        const int u = __shfl_up(v, o, 64);
-        if (tid >= o) v += u;
-      }
-      if (e < E) eoff[e + 1] = carry + v;
-      carry += __shfl(v, 63, 64);
-    }
+    if (lane == 63) wsum[wv] = v;
+    __syncthreads();
+    for (int w = 0; w < wv; w++) v += wsum[w];
+    if (tid < E) eoff[tid + 1] = v;
     if (tid == 0) eoff[0] = 0;
   }
   __syncthreads();
   const int total = eoff[E];
-  // pass 2: place every slot; the group's first lane advances the running count
-  for (int cb = c0; cb < c1; cb += KB) {
-    int ev[KB];
-    load_ids(cb, ev);
-#pragma unroll
-    for (int q = 0; q < KB; q++) {
-      if (cb + q >= c1) break;
-      const int e = ev[q];
-      const uint64_t m = same_expert(e, nbits);
-      const int rank = __popcll(m & below);
-      if (e >= 0) sorted[eoff[e] + mine[e] + rank] = (cb + q) * 64 + lane;
-      __builtin_amdgcn_wave_barrier();  // every lane has read mine[e] before it moves
-      if (e >= 0 && rank == 0) mine[e] += __popcll(m);
-      __builtin_amdgcn_wave_barrier();
-    }
+  // this workgroup's share of the padding, the tail and the expert ids
+  for (int i = tid; i < (E + G - 1) / G * bs && !none; i += kAlignThreads) {
+    const int e = g + i / bs * G;
+    if (e >= E) break;
+    const int p = eoff[e] + before[e] + rest[e] + i % bs;
+    if (p < eoff[e + 1]) sorted[p] = pad;
   }
-  // expert of every padded block: the e with eoff[e] <= b*bs < eoff[e+1]
-  for (int b = tid; b < total / bs; b += kAlignThreads) {
-    int lo = 0, hi = E;  // find last e with eoff[e] <= b*bs
+  for (int i = total + g * kAlignThreads + tid; i < max_padded; i += G * kAlignThreads) sorted[i] = pad;
+  for (int b = g * kAlignThreads + tid; b < max_blocks; b += G * kAlignThreads) {
+    int lo = 0, hi = E;  // expert of block b: the last e with eoff[e] <= b*bs
     const int v = b * bs;
     while (hi - lo > 1) {
       const int mid = (lo + hi) >> 1;
       if (eoff[mid] <= v) lo = mid; else hi = mid;
     }
-    experts[b] = emap ? emap[lo] : lo;
+    experts[b] = v >= total ? 0 : emap ? emap[lo] : lo;
   }
-  if (tid == 0) ntpp[0] = total;
+  if (g == 0 && tid == 0) {
+    ntpp[0] = total;
+    if (none) g_device_error = UB_ERR_INDEX;
+  }
+  if (none) return;
+  __syncthreads();  // `before` is read above and moves below
+  const uint64_t below = (1ull << lane) - 1;
+  for (int c0 = s0; c0 < s1; c0 += kAlignThreads) {
+    const int i = c0 + tid, e = i < s1 ? ids[i] : -1;
+    const uint64_t m = same_expert(e, nbits);
+    const int rank = __popcll(m & below);
+    if (e >= 0 && rank == 0) cnt[wv * E + e] = (uint16_t)__popcll(m);
+    __syncthreads();
+    if (e >= 0) {
+      int at = eoff[e] + before[e] + rank;
+      for (int w = 0; w < wv; w++) at += cnt[w * E + e];
+      sorted[at] = i;
+    }
+    if (c0 + kAlignThreads < s1) {
+      __syncthreads();
+      for (int x = tid; x < E; x += kAlignThreads) {
+        int sum = 0;
+        for (int w = 0; w < kAlignWaves; w++) sum += cnt[w * E + x], cnt[w * E + x] = 0;
+        before[x] += sum;
+      }
+      __syncthreads();
+    }
+  }
 }
 
 // ======================================== moe_align for small slot counts
 // The same outputs as k_moe_align (no expert_map / real_token_num), for
-// n = T*k <= 4096 slots in one workgroup of 1024 threads.  Slots are cut
+// n = T*k <= 1024 slots in one workgroup of 1024 threads (8 / 256 / 1024 slots
+// of 128 experts 4.8 / 5.0 / 6.0 us, k_moe_align 5.8 / 5.9 / 6.4; at 2048 7.0
+// and 6.1).  Slots are cut
 // into chunks of 64, one wavefront-wide chunk per (wave, q).  Within a chunk
 // the lanes holding the same expert are found by one ballot per bit of the
 // expert id (log2 E ballots), so a slot's rank among equal experts before it
@@ -372,7 +377,7 @@ __global__ void __launch_bounds__(kAlignThreads) k_moe_align(
 // position is eoff[e] + (slots of e in earlier chunks) + rank: ascending
 // slot order within each expert, as the reference.  No loop over the slots
 // is serial.
-constexpr int kRouteThreads = 1024, kRouteWaves = kRouteThreads / 64, kRouteMaxN = 4096;
+constexpr int kRouteThreads = 1024, kRouteWaves = kRouteThreads / 64, kRouteMaxN = 1024;
 constexpr int kRouteQ = kRouteMaxN / 64 / kRouteWaves;  // chunks per wave
 
 // The align, by the whole 1024-thread workgroup; ids in global memory or
@@ -1109,12 +1114,16 @@ static int moe_align_launch(int* sorted_ids, int* experts_ids, int* num_tokens_p
                        num_experts, block_size, ub_stream(stream));
     return ub_check_launch(nm);
   }
-  const size_t lds = sizeof(int) * ((size_t)(kAlignWaves + 1) * num_experts + 1);
+  // one wavefront-wide chunk per wavefront and workgroup, up to a workgroup per CU
+  const size_t lds = align_lds(num_experts);
+  const long slots = (long)token_num * topk;
+  const int groups = (int)std::max<long>(1, std::min<long>((slots + kAlignThreads - 1) / kAlignThreads, 256));
+  const int run = (int)((slots + (long)groups * kAlignThreads - 1) / ((long)groups * kAlignThreads)) * kAlignThreads;
   (void)hipFuncSetAttribute((const void*)k_moe_align, hipFuncAttributeMaxDynamicSharedMemorySize,
                       (int)lds);
-  k_moe_align<<<1, kAlignThreads, lds, ub_stream(stream)>>>(
+  k_moe_align<<<groups, kAlignThreads, lds, ub_stream(stream)>>>(
       sorted_ids, experts_ids, num_tokens_post_pad, topk_ids, real_token_num, expert_map,
-      num_experts, block_size, token_num, topk);
+      num_experts, block_size, token_num, topk, run);
   return ub_check_launch(nm);
 }
 
