@@ -564,6 +564,40 @@ def test_pipelined_k_split_over_workgroups(dev, M):
         assert (split == whole).float().mean().item() > 0.9
 
 
+@pytest.mark.parametrize("bits,rhs_t", [(4, 0), (8, 0), (8, 1)])
+@pytest.mark.parametrize("M,K,N", [(40, 192, 264), (130, 192, 64), (33, 704, 1000), (150, 3520, 520),
+                                   (64, 8256, 72), (300, 960, 776)])
+def test_pipelined_uneven_k_split(dev, bits, rhs_t, M, K, N):
+    # odd numbers of 64-k steps (the upper K-half then has one step past K) and
+    # parts of different lengths, against f64; a row of NaN and one of
+    # infinities touch no other row
+    a, w, sc, zt, a32, wd = _quant_case(bits, rhs_t, M, K, N, 64, torch.bfloat16, M + K + bits)
+    a = a.clone()
+    a[7], a[M - 1] = float("nan"), float("inf")
+    got = ops.matmul_quant(a, w, sc, zt, bits=bits, group_size=64, rhs_transpose=bool(rhs_t))
+    want = a32.astype(np.float64) @ wd.astype(np.float64)
+    keep = [m for m in range(M) if m not in (7, M - 1)]
+    got = got.float().cpu().numpy().astype(np.float64)
+    assert np.isnan(got[7]).all() and not np.isfinite(got[M - 1]).any()
+    # one bf16 rounding of an f32 sum (error far below it)
+    rms = np.sqrt(np.mean(want[keep] ** 2))
+    assert np.all(np.abs(got[keep] - want[keep]) <= 2.0**-8 * np.abs(want[keep]) + 1e-4 * rms)
+
+
+@pytest.mark.parametrize("qt", [ops.Q4_0, ops.Q8_0, ops.Q4_K])
+@pytest.mark.parametrize("M,K,N", [(64, 1280, 40), (41, 14336, 72), (200, 2816, 520)])
+def test_qmatmul_uneven_k_split(dev, qt, M, K, N):
+    # parts that start inside a 256-k span (whose headers serve four K-steps):
+    # f32 outputs against f64 of the dequantized bf16 weights
+    w = torch.from_numpy(synth.make_weight_soa(qt, N, K, seed=M)).to(dev)
+    x = torch.randn(M, K, device=dev, generator=torch.Generator(device=dev).manual_seed(K)).bfloat16()
+    y = ops.QMatMul(qt, w, N, K)(x)
+    wd = ops.dequantize_block(qt, w, N * K, torch.bfloat16).view(N, K)
+    want = x.double() @ wd.double().t().contiguous()
+    rms = want.square().mean().sqrt()
+    assert bool(((y.double() - want).abs() <= 1e-5 * want.abs() + 1e-5 * rms).all())
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("M", [128, 40])
 def test_pipelined_dequant_bit_exact(dev, dtype, M):

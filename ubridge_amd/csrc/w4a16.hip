@@ -40,6 +40,8 @@
 #include "common.h"
 #include "lds_dma.h"
 
+#include <algorithm>
+
 namespace {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -147,8 +149,8 @@ struct W4Args {
   void* c;
   int M, N, K, group;
   int c_f32;    // C is f32 (else T)
-  int ksplit;   // > 1: workgroup (tile, blockIdx.y) takes K-steps [y, y + 1) K / 64 / ksplit
-  float* part;  // and stores its f32 partial sums to part[y][M][N] (summed by k_ksum)
+  int ksplit;   // > 1: workgroup (tile, blockIdx.y) takes the y-th of ksplit nearly equal runs
+  float* part;  // of K-steps and stores its f32 partial sums to part[y][M][N] (summed by k_ksum)
 };
 
 // LDS image of one K-step (64 k) of the weight for 256 columns.
@@ -230,8 +232,14 @@ __global__ void __launch_bounds__(64 * NV) __attribute__((amdgpu_waves_per_eu(NV
   const int n0 = tile_n * kBN, m0 = tile_m * BM;
   const int M = p.M, N = p.N, K = p.K;
   const int S = p.ksplit > 1 ? p.ksplit : 1;
-  const int nkh = K / 64 / S / KS;             // K-steps per K-half
-  const int kb = blockIdx.y * (K / 64 / S);    // first K-step of this workgroup
+  // This workgroup's run of units of KS K-steps: nkh steps per K-half from
+  // step kb.  With KS = 2 and an odd number of steps the last step of the
+  // upper half lies past K: its A rows are loaded as zeros (`past`; the scales
+  // there, and with them the weights, read as zero too).
+  const int units = (K / 64 + KS - 1) / KS;
+  const int u0 = (int)((long)units * blockIdx.y / S), u1 = (int)((long)units * (blockIdx.y + 1) / S);
+  const int nkh = u1 - u0, kb = u0 * KS;
+  const bool past = KS == 2 && u1 * KS > K / 64;
   const ub_u32x4 ra = ub_desc(p.a, (uint64_t)M * K * 2);
   const uint64_t wbytes = WF == kGptq ? (uint64_t)(K / 8) * N * 4
                           : WF == kU4 || kNib32(WF) ? (uint64_t)(K / 2) * N
@@ -319,7 +327,8 @@ __global__ void __launch_bounds__(64 * NV) __attribute__((amdgpu_waves_per_eu(NV
     for (int i = 0; i < NA; i++) {
       const int U = (i * NV + wave) * 64;
       const int h = U / (AB / 16), u0 = U % (AB / 16);
-      ub_lds_load16_at(ra, st + h * HB + u0 * 16, voA[i], (uint32_t)kt * 128u);
+      const uint32_t vo = KS == 2 && past && h == 1 && kt == nkh - 1 ? kDmaOOB : voA[i];
+      ub_lds_load16_at(ra, st + h * HB + u0 * 16, vo, (uint32_t)kt * 128u);
     }
 #pragma unroll
     for (int j = 0; j < NW; j++) {
@@ -835,12 +844,12 @@ int num_cus() {
   return n;
 }
 
-// Tile 256 x 256 (2 x 2 wavefronts) or 128 x 256 with K split over two
-// wavefront pairs: whichever keeps more of the CUs busy over the launch's
+// Tile 256 x 256 (2 x 2 wavefronts) or 128 x 256 with K (of at least two
+// K-steps, an odd number too) split over two wavefront pairs: whichever keeps more of the CUs busy over the launch's
 // rounds (ties: the taller tile, which reads half the weight per flop).
 // force: 0 shape rule, 1 split, 2 no split.
 bool pick_split(int M, int N, int K, int force) {
-  const bool can_split = K % 128 == 0;
+  const bool can_split = K >= 128;
   if (force == 1) return can_split;
   if (force == 2 || !can_split) return false;
   const long cus = num_cus(), tn = ub_cdiv(N, kBN);
@@ -869,19 +878,26 @@ int gemm_tile_force() {
 }
 
 // out[i] = sum over s = 0..S-1 of part[s][i], in that order (f32), as f32
-// (DT = UB_F32) or rounded once to T; 4 elements per thread, the S loads
-// unrolled so that they are all in flight together.
-template <int DT, int S>
-__global__ void __launch_bounds__(256) k_ksum(const float* __restrict__ part, size_t n4,
+// (DT = UB_F32) or rounded once to T; 4 elements per thread, eight loads in
+// flight at a time.
+template <int DT>
+__global__ void __launch_bounds__(256) k_ksum(const float* __restrict__ part, size_t n4, int S,
                                               void* __restrict__ out) {
   const size_t i = blockIdx.x * (size_t)256 + threadIdx.x;
   if (i >= n4) return;
-  float4 v[S];
+  float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
+  for (int s0 = 0; s0 < S; s0 += 8) {
+    float4 v[8];
 #pragma unroll
-  for (int s = 0; s < S; s++) v[s] = ((const float4*)part)[(size_t)s * n4 + i];
-  float4 a = v[0];
+    for (int s = 0; s < 8; s++)
+      if (s0 + s < S) v[s] = ((const float4*)part)[(size_t)(s0 + s) * n4 + i];
 #pragma unroll
-  for (int s = 1; s < S; s++) a.x += v[s].x, a.y += v[s].y, a.z += v[s].z, a.w += v[s].w;
+    for (int s = 0; s < 8; s++)
+      if (s0 + s < S) {
+        if (s0 + s == 0) a = v[0];
+        else a.x += v[s].x, a.y += v[s].y, a.z += v[s].z, a.w += v[s].w;
+      }
+  }
   if constexpr (DT == UB_F32) {
     ((float4*)out)[i] = a;
   } else {
@@ -894,22 +910,22 @@ __global__ void __launch_bounds__(256) k_ksum(const float* __restrict__ part, si
 }
 
 // Split over K across workgroups for grids that leave CUs idle: with fewer
-// tiles than half the CUs, each tile's K range is cut in S = 2, 4 or 8 parts
-// (tiles x S <= CUs), the parts' f32 sums go to the stream's workspace and
-// k_ksum adds them in a fixed order.  S = 1 where K does not divide (the
-// GGUF formats: whole 256-k spans per part) or the call may not allocate
-// (may_alloc false: the allocation-free entry point).
-// MI355X, 4096 x 14336 GPTQ at 64 / 256 tokens: 56 / 112 tiles.
-int pick_ksplit(const W4Args& p, bool split, bool gguf, bool may_alloc) {
+// tiles than half the CUs, each tile's K-steps are cut in S nearly equal
+// parts, as many as the CUs take (tiles x S <= CUs); the parts' f32 sums go to
+// the stream's workspace and k_ksum adds them in a fixed order.  S up to 8, and
+// up to 16 where a part keeps at least 4 units of K-steps (beyond, the longer
+// sum costs what the shorter walk gives: 24 x 4096 x 4096 GPTQ at S = 8 / 16
+// 14.4 / 15.3 us, but 24 x 14336 x 4096 25.7 / 20.7, 64 tokens 28.3 / 25.2,
+// Q4_K 34.5 / 28.4).  S = 1 where the call may not allocate (may_alloc false:
+// the allocation-free entry point).  Parts need not be equal: int8 [N, K] 201
+// x 3520 x 9000 (36 tiles of 256 x 256 or 72 of 128 x 256, 55 K-steps) 89 us
+// unsplit, 39 as 72 tiles x 3.
+int pick_ksplit(const W4Args& p, bool split, bool may_alloc) {
   if (!may_alloc || ub_tune(UB_TUNE_W4A16_PATH) == 7) return 1;
-  const int KS = split ? 2 : 1;
+  const int units = split ? ub_cdiv(p.K, 128) : p.K / 64;
   const long tiles = (long)ub_cdiv(p.M, split ? (small_tiles(p.M) ? 64 : 128) : 256) * ub_cdiv(p.N, kBN);
-  const long cus = num_cus();
-  int S = 1;
-  while (S < 8 && tiles * S * 2 <= cus && (p.K / 64) % (S * 2 * KS) == 0 &&
-         (!gguf || (p.K / 256) % (S * 2) == 0))
-    S *= 2;
-  return S;
+  const int most = std::min(units, std::max(8, std::min(16, units / 4)));
+  return (int)std::max<long>(1, std::min<long>(most, num_cus() / tiles));
 }
 
 // Scratch for the K split picked above (none when S == 1); sets p.ksplit and
@@ -926,14 +942,9 @@ int ksum_launch(const W4Args& p, int out_dt, hipStream_t s) {
   if (p.ksplit <= 1) return UB_OK;
   const size_t n4 = (size_t)p.M * p.N / 4;
   const unsigned g = (unsigned)((n4 + 255) / 256);
-#define UB_KS(DT)                                                                  \
-  if (p.ksplit == 2) k_ksum<DT, 2><<<g, 256, 0, s>>>(p.part, n4, p.c);             \
-  else if (p.ksplit == 4) k_ksum<DT, 4><<<g, 256, 0, s>>>(p.part, n4, p.c);        \
-  else k_ksum<DT, 8><<<g, 256, 0, s>>>(p.part, n4, p.c);
-  if (out_dt == UB_F32) { UB_KS(UB_F32) }
-  else if (out_dt == UB_F16) { UB_KS(UB_F16) }
-  else { UB_KS(UB_BF16) }
-#undef UB_KS
+  if (out_dt == UB_F32) k_ksum<UB_F32><<<g, 256, 0, s>>>(p.part, n4, p.ksplit, p.c);
+  else if (out_dt == UB_F16) k_ksum<UB_F16><<<g, 256, 0, s>>>(p.part, n4, p.ksplit, p.c);
+  else k_ksum<UB_BF16><<<g, 256, 0, s>>>(p.part, n4, p.ksplit, p.c);
   return ub_check_launch("w4a16 k-split sum");
 }
 
@@ -952,7 +963,7 @@ int ub_w4a16_pipelined(const void* a, const int32_t* qw, const void* scales, con
     return UB_ERR_UNSUPPORTED;  // 32-bit buffer offsets
   W4Args p{a, qw, scales, qzeros, out, M, N, K, group};
   const bool split = pick_split(M, N, K, gemm_tile_force());
-  KSplit ks(p, pick_ksplit(p, split, false, true), s);
+  KSplit ks(p, pick_ksplit(p, split, true), s);
   const int e = dispatch_wf<kGptq>(p, dtype, split, s);
   return e ? e : ksum_launch(p, dtype, s);
 }
@@ -974,7 +985,7 @@ int ub_wq_pipelined(int wf, const void* a, const void* w, const void* scales, co
     return UB_ERR_UNSUPPORTED;  // 32-bit buffer offsets
   W4Args p{a, w, scales, zeros, out, M, N, K, group};
   const bool split = pick_split(M, N, K, tile ? tile : gemm_tile_force());
-  KSplit ks(p, pick_ksplit(p, split, false, true), s);
+  KSplit ks(p, pick_ksplit(p, split, true), s);
   const int e = wf == kU4    ? dispatch_wf<kU4>(p, dtype, split, s)
                 : wf == kI8Kn ? dispatch_wf<kI8Kn>(p, dtype, split, s)
                               : dispatch_wf<kI8Nk>(p, dtype, split, s);
@@ -1004,7 +1015,7 @@ int ub_gguf_pipelined(int qtype, const void* w, const void* x, void* y, int y_f3
   const uint8_t* hdr = (const uint8_t*)w;
   W4Args p{x, hdr + hdr_b, nullptr, hdr, y, M, N, K, 256, y_f32};
   const bool split = pick_split(M, N, K, gemm_tile_force());
-  KSplit ks(p, pick_ksplit(p, split, true, may_alloc), s);
+  KSplit ks(p, pick_ksplit(p, split, may_alloc), s);
   const int e = qtype == UB_Q4_K   ? dispatch_wf<kQ4K>(p, UB_BF16, split, s)
                 : qtype == UB_Q8_0 ? dispatch_wf<kQ8_0>(p, UB_BF16, split, s)
                                    : dispatch_wf<kQ4_0>(p, UB_BF16, split, s);
