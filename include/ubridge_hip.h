@@ -355,6 +355,12 @@ int ubridge_fused_moe_w8a16_silu(void* C, const void* A, const int8_t* B, const 
                                  const int* num_tokens_post_pad, int M, int K, int N, int E,
                                  int topk_ids_size, int top_k, int block_size, int bias_flag,
                                  int dtype, void* stream);
+/* the same for 16-bit experts (B in A's dtype). */
+int ubridge_fused_moe_silu(void* C, const void* A, const void* B, const void* bias,
+                           const int* sorted_ids, const int* experts_ids,
+                           const int* num_tokens_post_pad, int M, int K, int N, int E,
+                           int topk_ids_size, int top_k, int block_size, int bias_flag,
+                           int dtype, void* stream);
 
 /* out[T, d] = silu(x[T, :d]) * x[T, d:] and out[T, N] = sum_k in[T, k, N]:
  * the activation and combine steps between the two expert GEMMs. */

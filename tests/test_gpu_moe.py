@@ -452,6 +452,33 @@ def test_fused_gate_up_silu_matches_two_calls(dev, T, k, E, K, I, bs, dtype, ema
     assert torch.equal(got.view(torch.int16), want.view(torch.int16))
 
 
+@pytest.mark.parametrize("path", [0, 10])
+@pytest.mark.parametrize("T,k,E,K,I,bs,dtype,q8", [
+    (37, 3, 8, 448, 72, 16, torch.bfloat16, False), (300, 2, 3, 192, 200, 32, torch.float16, False),
+    (1030, 4, 16, 128, 1284, 32, torch.bfloat16, False),  # the tiles without the knob
+    (300, 2, 3, 192, 204, 64, torch.float16, True), (37, 3, 8, 448, 72, 16, torch.bfloat16, True)])
+def test_gate_up_silu_tiles_and_16_bit(dev, moe_path, path, T, k, E, K, I, bs, dtype, q8):
+    g = torch.Generator().manual_seed(T + I)
+    ids = torch.randint(0, E, (T, k), generator=g, dtype=torch.int32)
+    s, e, n = moe.moe_align_block_size(ids.to(dev), E, bs)
+    x = torch.randn(T, K, generator=g).to(dtype).to(dev)
+    if q8:
+        w13 = torch.randint(-127, 128, (E, 2 * I, K), generator=g, dtype=torch.int8).to(dev)
+        s13 = (torch.rand(E, 2 * I, generator=g) * 0.01 + 0.001).to(dtype).to(dev)
+    else:
+        w13, s13 = (torch.randn(E, 2 * I, K, generator=g) * 0.1).to(dtype).to(dev), None
+    bias = torch.randn(E, 2 * I, generator=g).to(dtype).to(dev)
+    moe_path(path)
+    h1 = torch.zeros(T * k, 2 * I, dtype=dtype, device=dev)
+    moe.invoke_fused_moe(x, w13, h1, None, s, e, n, k, bs, False, B_scale=s13, bias=bias)
+    want = moe.silu_and_mul(h1)
+    got = torch.full((T * k + 1, I), 7.0, dtype=dtype, device=dev)
+    moe.fused_moe_gate_up_silu(x, w13, s13, s, e, n, k, bs, bias=bias, out=got[:T * k],
+                               topk_ids_size=T * k)
+    assert torch.equal(got[:T * k].view(torch.int16), want.view(torch.int16))
+    assert bool((got[T * k] == 7.0).all())
+
+
 @pytest.mark.parametrize("N,dtype", [(40, torch.bfloat16), (36, torch.bfloat16), (2048, torch.float16)])
 def test_moe_sum_bits(dev, N, dtype):
     # f32 accumulation in slot order, one rounding: bit for bit (the 8-column
