@@ -188,6 +188,7 @@ def moe_path():
     ops.tune_set("moe_gemm_path", 0)
 
 
+@pytest.mark.parametrize("path", [10, 11, 12])  # tiles of 128, 64, 32 (int8) rows
 @pytest.mark.parametrize("K,N,bs,q8,mrw,bias,emap,dtype", [
     (64, 8, 32, True, 0, False, False, torch.bfloat16),      # one K-step, one column block's edge
     (128, 264, 32, True, 1, True, True, torch.bfloat16),     # partial column block, -1 and shared experts
@@ -195,8 +196,8 @@ def moe_path():
     (320, 256, 64, False, 0, True, False, torch.float16),
     (64, 48, 128, True, 1, False, False, torch.float16),
     (448, 72, 1, False, 0, False, True, torch.bfloat16)])
-def test_moe_tile_kernel(dev, moe_path, K, N, bs, q8, mrw, bias, emap, dtype):
-    # 128-row tiles: experts with 0, 1, 31 .. 33, 95 .. 97, 127 .. 129, 300
+def test_moe_tile_kernel(dev, moe_path, path, K, N, bs, q8, mrw, bias, emap, dtype):
+    # experts with 0, 1, 31 .. 33, 95 .. 97, 127 .. 129, 300
     # rows, against f64, rows of experts mapped to -1 zeroed, everything past
     # the slots untouched
     rows = [0, 1, 31, 32, 33, 0, 64, 65, 95, 96, 97, 127, 128, 129, 300, 2]
@@ -223,7 +224,7 @@ def test_moe_tile_kernel(dev, moe_path, K, N, bs, q8, mrw, bias, emap, dtype):
     bv = torch.randn(E, N, generator=g).to(dtype).to(dev) if bias else None
     tw = torch.rand(T * k, generator=g).to(dev)
     C = torch.full((T * k + 1, N), 3.0, dtype=dtype, device=dev)
-    moe_path(10)
+    moe_path(path)
     moe.invoke_fused_moe(A, B, C[:T * k], tw if mrw else None, s, e, n, k, bs, mrw, B_scale=Bs,
                          bias=bv)
     ex = ids.flatten().long() if em is None else em.long()[ids.flatten().long()]
@@ -254,11 +255,12 @@ def test_moe_tile_windows(dev, moe_path):
     A = torch.randn(ids.shape[0], K, generator=g).bfloat16().to(dev)
     B = torch.randn(E, N, K, generator=g).bfloat16().to(dev)
     out = []
-    for path in (1, 10):
+    for path in (1, 10, 11):
         moe_path(path)
         C = torch.zeros(ids.shape[0], N, dtype=torch.bfloat16, device=dev)
         out.append(moe.invoke_fused_moe(A, B, C, None, s, e, n, k, 32, False))
     assert torch.equal(out[0].view(torch.int16), out[1].view(torch.int16))
+    assert torch.equal(out[0].view(torch.int16), out[2].view(torch.int16))
 
 
 def test_moe_tile_bad_expert_flagged(dev, moe_path):
@@ -452,7 +454,7 @@ def test_fused_gate_up_silu_matches_two_calls(dev, T, k, E, K, I, bs, dtype, ema
     assert torch.equal(got.view(torch.int16), want.view(torch.int16))
 
 
-@pytest.mark.parametrize("path", [0, 10])
+@pytest.mark.parametrize("path", [0, 10, 11, 12])
 @pytest.mark.parametrize("T,k,E,K,I,bs,dtype,q8", [
     (37, 3, 8, 448, 72, 16, torch.bfloat16, False), (300, 2, 3, 192, 200, 32, torch.float16, False),
     (1030, 4, 16, 128, 1284, 32, torch.bfloat16, False),  # the tiles without the knob

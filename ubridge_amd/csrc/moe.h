@@ -21,8 +21,9 @@ struct MoeArgs {
   int a_div;  // slot s reads A row s / a_div
 };
 
-// The grouped GEMM on 128-row tiles (moe_tile.hip); err: the device flag of
-// out-of-range expert ids.  false: nothing launched, the call is outside its
-// contract.  ub_moe_tile_pays: whether the sizes are those it is faster at.
-bool ub_moe_tile(const MoeArgs& a, int dt, bool q8, int* err, hipStream_t s);
-bool ub_moe_tile_pays(const MoeArgs& a, bool q8);
+// The grouped GEMM on tiles of 32 (int8 only), 64 or 128 rows (moe_tile.hip);
+// err: the device flag of out-of-range expert ids.  false: nothing launched,
+// the call is outside its contract.  ub_moe_tile_rows: the rows to take for
+// these sizes, 0 where k_moe_gemm is faster.
+bool ub_moe_tile(const MoeArgs& a, int rows, int dt, bool q8, int* err, hipStream_t s);
+int ub_moe_tile_rows(const MoeArgs& a, bool q8);

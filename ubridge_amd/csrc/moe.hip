@@ -836,11 +836,14 @@ __global__ void __launch_bounds__(64 * NWV) k_moe_gemm(MoeArgs a) {
 // 2: 256 columns, BK 64, 4 stages; 3: 128 columns, BK 64, 6 stages;
 // 4: 256 columns, BK 128, 3 stages (int8 only); 5: 128 columns, BK 64,
 // 4 stages; 6 / 7: 64 columns, BK 64, 4 / 6 stages; 8: 128 columns, BK 64,
-// 3 stages; 9: 64 columns, BK 128, 3 stages; 10: the 128-row tiles of
-// moe_tile.hip.  Automatic (0): 10 where ub_moe_tile_pays, else 1 for int8
-// experts with K >= 1536 and for 16-bit experts, else 8 -- measured on
-// MI355X at the Qwen3-MoE shapes (gate/up K = 2048, down K = 768), where
-// both stream within ~2% of the same ring with the MFMA work removed.
+// 3 stages; 9: 64 columns, BK 128, 3 stages; 10 / 11 / 12: the 128-, 64- and
+// (int8) 32-row tiles of moe_tile.hip.  Automatic (0): those where
+// ub_moe_tile_rows says so, else 1 while its workgroups (about one block per
+// expert in use and 32 slots, times the column blocks) fit the CUs at once, two
+// per CU, and 8 (half the LDS, four per CU) beyond: 128 experts, int8 gate/up +
+// down, us with 1 / 8: 1 token 28.0 / 32.5, 8 tokens 66 / 60, 32 tokens 116 /
+// 108; 16-bit 8 tokens 114 / 109, 32 tokens 209 / 193; 8 experts, 128 tokens,
+// int8 51.8 / 57.7.
 // (Weights loaded straight into MFMA-operand registers measured slower:
 // 32 lanes x 32 contiguous bytes per instruction streams ~17% below the
 // 128-byte row runs of the direct-to-LDS loads.)
@@ -851,7 +854,10 @@ void moe_gemm_launch(int path, const MoeArgs& a, int max_blocks, hipStream_t s) 
               ub_cdiv(a.bs, MBM));
     kern<<<grid, 64 * nwv, 0, s>>>(a);
   };
-  if (path == 0) path = !Q8 || a.K >= 1536 ? 1 : 8;
+  if (path == 0) {
+    const long blocks = std::min<long>(a.tis, a.E) + a.tis / MBM;
+    path = blocks * ub_cdiv(a.act ? a.N / 2 : a.N, a.act ? 64 : 128) <= 512 ? 1 : 8;
+  }
   switch (path) {
     case 2: go(k_moe_gemm<DT, Q8, 8, 64, 4>, 8); break;
     case 3: go(k_moe_gemm<DT, Q8, 4, 64, 6>, 4); break;
@@ -910,9 +916,8 @@ int moe_gemm(const char* nm, int dt, bool q8, void* C, const void* A, const void
   const int max_blocks = (tis + E * (bs - 1)) / bs;
   hipStream_t s = ub_stream(stream);
   const int path = ub_tune(UB_TUNE_MOE_GEMM_PATH);
-  if ((path == 10 || (path == 0 && ub_moe_tile_pays(a, q8))) &&
-      ub_moe_tile(a, dt, q8, error_flag(), s))
-    return ub_check_launch(nm);
+  const int rows = path == 0 ? ub_moe_tile_rows(a, q8) : path == 10 ? 128 : path == 11 ? 64 : path == 12 && q8 ? 32 : 0;
+  if (rows && ub_moe_tile(a, rows, dt, q8, error_flag(), s)) return ub_check_launch(nm);
   if (dt == UB_BF16) {
     if (q8) moe_gemm_launch<UB_BF16, true>(path, a, max_blocks, s);
     else moe_gemm_launch<UB_BF16, false>(path, a, max_blocks, s);

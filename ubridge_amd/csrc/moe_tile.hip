@@ -1,5 +1,5 @@
-// moe_tile.hip -- grouped expert GEMM on 128-row tiles, for batches whose
-// experts get many rows each (gfx950).
+// moe_tile.hip -- grouped expert GEMM on tiles of 32, 64 or 128 rows, for
+// batches that fill them (gfx950).
 //
 // The same operation as k_moe_gemm (moe.hip), which gives every sorted block
 // of 32 rows its own workgroup per column tile: a stream of the weights while
@@ -7,20 +7,21 @@
 // blocks, and then each of them fetches the expert's weights again, widens
 // every int8 weight again for a single row of MFMA tiles, and fills one 32 x
 // 32 tile per wavefront.  Here the blocks of one expert are taken together in
-// tiles of up to 128 rows, so one widened weight fragment feeds up to 4 MFMAs
-// and the weights are fetched a quarter as often.
+// tiles of kTM = 32, 64 or 128 rows, so one widened weight fragment feeds up
+// to 4 MFMAs and the weights are fetched a quarter as often; with few rows (32)
+// what is left is the persistent grid, whose loads do not stop between tiles.
 //
 //  * Persistent grid, two workgroups of 4 wavefronts per CU (so the two
 //    wavefronts of a SIMD are not held in step by one barrier; one workgroup
 //    of 8 measured 1-10% slower).  Each workgroup first cuts the sorted
 //    blocks into tiles itself (two scans over experts_ids; consecutive
-//    blocks of one expert, at most 128 rows) and keeps the list in LDS, then
+//    blocks of one expert, at most kTM rows) and keeps the list in LDS, then
 //    walks (tile, column block) pairs.
-//  * Tile 128 rows x 256 weight rows; a wavefront owns 64 weight rows and
-//    all 128 token rows: 4 x 2 tiles of v_mfma_f32_32x32x16.  A lane's two
+//  * Tile kTM rows x 256 weight rows; a wavefront owns 64 weight rows and
+//    all token rows: up to 4 x 2 tiles of v_mfma_f32_32x32x16.  A lane's two
 //    columns are adjacent, so a store covers 128-byte runs of two rows.
 //    Tiles with at most 96 / 64 / 32 rows run the loop with 3 / 2 / 1 row
-//    tiles.  With the gated output a wavefront's two column tiles are the
+//    tiles of 32.  With the gated output a wavefront's two column tiles are the
 //    gate and the up rows of the same 32 columns, so silu(g) u is lane-local.
 //  * Both operands reach LDS by direct-to-LDS loads through a ring of NS
 //    K-step stages (A rows gathered by slot), XOR-swizzled in 16-byte units;
@@ -34,7 +35,7 @@
 //    sums as in k_moe_gemm.
 //
 // MI355X, 128 experts of 2048 -> 2 x 768 -> 2048, top-8, us (k_moe_gemm /
-// this), int8 at 1024 tokens: gate/up 194 / 125, down 100 / 75; at 4096: 587 /
+// 128-row tiles), int8 at 1024 tokens: gate/up 194 / 125, down 100 / 75; at 4096: 587 /
 // 271, 301 / 165 (760 / 626 TFLOP/s); bf16 at 1024: 263 / 212, 205 / 110; at
 // 4096: 751 / 348, 704 / 198.  At 4096 int8 tokens the gate/up launch without
 // its epilogue takes 25 us less, with every load an L2 hit 34 us less, without
@@ -52,7 +53,6 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-constexpr int kTM = 128;     // rows of a tile
 constexpr int NWV = 4, kCols = 64 * NWV;  // wavefronts, weight rows of a workgroup
 constexpr int kTiles = 512;  // tiles listed in LDS at a time
 constexpr uint16_t kElsewhere = 0xffff, kBadExpert = 0xfffe;  // list entries without weights here
@@ -114,15 +114,17 @@ __device__ __forceinline__ uint4 i8x8_to_t(uint32_t lo, uint32_t hi) {
   return make_uint4(o[0], o[1], o[2], o[3]);
 }
 
-template <int DT, bool Q8, int BK, int NS>
+template <int DT, bool Q8, int kTM, int BK, int NS>
 __global__ void __launch_bounds__(64 * NWV) __attribute__((amdgpu_waves_per_eu(2, 2)))
 k_moe_tile(MoeArgs a, int* err) {
   constexpr int NT = 64 * NWV, BN = kCols, SS = BK / 16;
   constexpr int WB = Q8 ? 1 : 2;
   constexpr int RA = BK * 2, UA = RA / 16;    // A row bytes / 16-byte units
   constexpr int RB = BK * WB, UB = RB / 16;   // weight row bytes / units
-  constexpr int AB = kTM * RA, BB = BN * RB, STB = AB + BB;
+  constexpr int AR = kTM * RA < 1024 * NWV ? 1024 * NWV / RA : kTM;  // A rows in LDS: a load per wave
+  constexpr int AB = AR * RA, BB = BN * RB, STB = AB + BB;
   constexpr int NA = AB / 1024 / NWV, NB = BB / 1024 / NWV, NL = NA + NB;  // loads per wave, stage
+  static_assert(kTM == 128 || kTM == 64 || kTM == 32, "rows of a tile");
   static_assert(AB % (1024 * NWV) == 0 && BB % (1024 * NWV) == 0, "loads split evenly");
   static_assert(Q8 ? BK == 64 : BK == 32, "substep schedule");
   constexpr int RPWA = RA >= 256 ? 1 : 256 / RA, RPWB = RB >= 256 ? 1 : 256 / RB;
@@ -277,14 +279,15 @@ k_moe_tile(MoeArgs a, int* err) {
     const int e = tab_e[q / ncol], n0 = (q % ncol) * CT;
     // rows up to the last real one (padding may lie before it, where two
     // neighbouring experts are mapped to the same weights)
-    const uint64_t lo = __ballot(srow[buf][lane] >= 0), hi = __ballot(srow[buf][64 + lane] >= 0);
+    const uint64_t lo = __ballot(lane < kTM && srow[buf][lane] >= 0);
+    const uint64_t hi = kTM > 64 ? __ballot(srow[buf][64 % kTM + lane] >= 0) : 0;
     const int nreal = hi ? 128 - __clzll(hi) : lo ? 64 - __clzll(lo) : 0;
     if (e >= a.E || nreal == 0) return 0;
     rb = ub_desc((const uint8_t*)a.B + (size_t)e * N * brow, (uint64_t)N * brow);
 #pragma unroll
     for (int j = 0; j < NA; j++) {
       const int u = (j * NWV + wave) * 64 + lane, r = u / UA, c = (u % UA) ^ swa(r);
-      const int s = srow[buf][r];
+      const int s = AR == kTM || r < kTM ? srow[buf][r % kTM] : -1;
       voA[j] = s >= 0 ? (uint32_t)(((size_t)(s / a.a_div) * K + 8 * c) * 2) : kDmaOOB;
     }
 #pragma unroll
@@ -342,7 +345,7 @@ k_moe_tile(MoeArgs a, int* err) {
       // wait for stage t + 1, free stage t for the loads of step t + NS
       auto turn = [&](int kt, uint32_t cur) {
         __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the reads of `cur` are done
-        if (NS == 3 && kt + 2 < nk) ub_wait_vmcnt<NL>();
+        if (NS > 2 && kt + NS - 1 < nk) ub_wait_vmcnt<(NS - 2) * NL>();
         else ub_wait_vmcnt<0>();
         ub_barrier();
         if (kt + NS < nk) issue(kt + NS, cur);
@@ -475,11 +478,18 @@ k_moe_tile(MoeArgs a, int* err) {
           }
       }
     };
-    if (nreal > 96) run(std::integral_constant<int, 4>{});
-    else if (nreal > 64) run(std::integral_constant<int, 3>{});
-    else if (nreal > 32) run(std::integral_constant<int, 2>{});
-    else if (nreal > 0) run(std::integral_constant<int, 1>{});
-    else {
+    auto rows = [&](auto tmc) {  // one loop per number of row tiles
+      if (nreal <= 32 * (decltype(tmc)::value - 1)) return false;
+      run(tmc);
+      return true;
+    };
+    bool done = false;
+    if constexpr (kTM == 128)
+      done = rows(std::integral_constant<int, 4>{}) || rows(std::integral_constant<int, 3>{}) ||
+             rows(std::integral_constant<int, 2>{});
+    if constexpr (kTM == 64) done = rows(std::integral_constant<int, 2>{});
+    if (!done) done = rows(std::integral_constant<int, 1>{});
+    if (!done) {
       __syncthreads();  // every wavefront is past the epilogue that reads the other row buffer
       const int e = tab_e[q / ncol];
       if (e == kElsewhere) {  // expert handled elsewhere (expert parallel): zero the rows
@@ -498,35 +508,45 @@ k_moe_tile(MoeArgs a, int* err) {
   }
 }
 
-template <int DT, bool Q8, int BK, int NS>
+template <int DT, bool Q8, int kTM, int BK, int NS>
 void launch(const MoeArgs& a, int* err, hipStream_t s) {
   const int NO = a.act ? a.N / 2 : a.N;
   const long pairs = (long)max_blocks(a) * ub_cdiv(NO, a.act ? kCols / 2 : kCols);  // at most
   const unsigned g = (unsigned)std::min<long>(ub_cdiv(pairs, 8) * 8, 512);
-  k_moe_tile<DT, Q8, BK, NS><<<g, 64 * NWV, 0, s>>>(a, err);
+  k_moe_tile<DT, Q8, kTM, BK, NS><<<g, 64 * NWV, 0, s>>>(a, err);
 }
 
 }  // namespace
 
-// Where the tiles pay, from sizes known on the host: an expert's average rows
-// r = slots / E and the (tile, column block) pairs, about slots / 128 + E / 2
-// tiles (at least one per expert).
-//  * int8 from r = 32: at r = 16 / 24 / 32 (256 / 384 / 512 tokens of the
-//    128-expert layer above) gate/up + down take 148 / 166 / 192 us in
-//    k_moe_gemm and 155 / 162 / 180 here (one row tile leaves the widening
-//    unshared and k_moe_gemm skips padding rows' loads).
-//  * 16-bit from r = 8: no widening; 128 tokens 267 / 254, 256 tokens 283 / 261.
-//  * at least 160 pairs: each walks all of K, so few of them leave the chip
-//    idle (8 experts 4096 -> 2 x 1024, top-2, int8 gate/up: 96 pairs 69 / 73,
-//    160 pairs 104 / 76, down 128 pairs 20.5 / 29, 192 pairs 33 / 28).
-bool ub_moe_tile_pays(const MoeArgs& a, bool q8) {
-  const long tiles = std::max<long>(a.E, a.tis / kTM + a.E / 2);
-  const long pairs = tiles * ub_cdiv(a.act ? a.N / 2 : a.N, a.act ? kCols / 2 : kCols);
-  return a.tis >= (long)a.E * (q8 ? 32 : 8) && pairs >= 160;
+// Rows of the tiles where they pay, 0 where k_moe_gemm is faster; from sizes
+// known on the host: an expert's average rows r = slots / E and the (tile,
+// column block) pairs, about slots / rows + E / 2 tiles (at least one per
+// expert).  Whole layers of 128 / 64 / 8 experts (top-8 2048 -> 2 x 768, top-6
+// 2048 -> 2 x 1408, top-2 4096 -> 2 x 1024), us:
+//  * taller tiles need rows to fill them.  int8, 128 experts, k_moe_gemm / 32 /
+//    64 / 128 rows at r = 2: 121 / 125 / - / 147, 4: 137 / 132 / 135 / 164, 16:
+//    163 / 163 / 169 / 181, 24: 180 / 170 / 172 / 184, 48: 243 / 218 / 199 /
+//    220, 96: 379 / - / 267 / 263, 128: 475 / - / 327 / 303; 64 experts at r =
+//    3: 121 / 119 / 121 / 146, 24: 163 / 153 / 151 / 179.  16-bit (no widening
+//    to share) k_moe_gemm / 64 / 128 rows at r = 4: 253 / 250 / 250, 8: 263 /
+//    261 / 261, 24: 286 / 280 / 279, 64: 404 / 336 / 348, 80: 467 / 389 / 347.
+//  * at least 160 pairs (128 int8 rows: 512): each walks all of K, so few of
+//    them leave the chip idle.  8 experts, int8 gate/up, k_moe_gemm / 32 / 64 /
+//    128 rows at r = 32 (96 / 64 / 64 pairs) 35 / 41 / 49 / 64, 64 (160 / 96 /
+//    64) 44 / 41 / 50 / 73, 128 (- / 160 / 96) 60 / 57 / 51 / 73, 256 (- / 288 /
+//    160) 100 / 85 / 70 / 78.
+int ub_moe_tile_rows(const MoeArgs& a, bool q8) {
+  const long cols = ub_cdiv(a.act ? a.N / 2 : a.N, a.act ? kCols / 2 : kCols);
+  auto pays = [&](int rows, int r, long pairs) {
+    return rows % a.bs == 0 && a.tis >= (long)a.E * r &&
+           std::max<long>(a.E, a.tis / rows + a.E / 2) * cols >= pairs;
+  };
+  if (q8) return pays(128, 112, 512) ? 128 : pays(64, 24, 160) ? 64 : pays(32, 3, 160) ? 32 : 0;
+  return pays(128, 8, 160) ? 128 : pays(64, 8, 160) ? 64 : 0;
 }
 
-bool ub_moe_tile(const MoeArgs& a, int dt, bool q8, int* err, hipStream_t s) {
-  if (!err || a.bs > kTM || kTM % a.bs != 0 || a.N % 8 != 0 || a.K % 64 != 0) return false;
+bool ub_moe_tile(const MoeArgs& a, int rows, int dt, bool q8, int* err, hipStream_t s) {
+  if (!err || rows % a.bs != 0 || a.N % 8 != 0 || a.K % 64 != 0) return false;
   // the list holds block and expert numbers in 16 bits
   if (max_blocks(a) >= 65535 || a.E >= kBadExpert) return false;
   if ((((uintptr_t)a.A | (uintptr_t)a.B) & 15) != 0 || ((uintptr_t)a.C & 3) != 0) return false;
@@ -535,8 +555,14 @@ bool ub_moe_tile(const MoeArgs& a, int dt, bool q8, int* err, hipStream_t s) {
     return false;  // 32-bit buffer offsets
   auto go = [&](auto dtc) {
     constexpr int DT = decltype(dtc)::value;
-    if (q8) launch<DT, true, 64, 2>(a, err, s);
-    else launch<DT, false, 32, 3>(a, err, s);
+    if (q8) {
+      if (rows == 128) launch<DT, true, 128, 64, 2>(a, err, s);
+      else if (rows == 64) launch<DT, true, 64, 64, 3>(a, err, s);
+      else launch<DT, true, 32, 64, 3>(a, err, s);
+    } else {
+      if (rows == 128) launch<DT, false, 128, 32, 3>(a, err, s);
+      else launch<DT, false, 64, 32, 3>(a, err, s);
+    }
   };
   if (dt == UB_BF16) go(std::integral_constant<int, UB_BF16>{});
   else go(std::integral_constant<int, UB_F16>{});
