@@ -605,3 +605,31 @@ def test_qmatmul_misaligned_bf16_x_gemm_sizes(dev, qt, M):
     assert torch.equal(y, y2)
     xf = torch.from_numpy(x).to(dev).to(torch.bfloat16).float().cpu().numpy()
     assert rel_err(got, oracle.qmatmul(qt, synth.make_weight_soa(qt, N, K, seed=qt), xf, N, K)) < 1e-2
+
+
+def test_qmatmul_forms_of_x_and_out(dev):
+    # x of one, two and three dimensions, a strided x, and results given in the
+    # (M, N) or another shape of as many values, on the current and a side stream
+    N, K = 64, 256
+    mm = ops.QMatMul(ops.Q4_0, torch.from_numpy(synth.make_weight_soa(ops.Q4_0, N, K, seed=3)).to(dev),
+                     N, K)
+    x = torch.randn(6, K, device=dev)
+    want = mm(x)
+    assert want.shape == (6, N) and want.dtype == torch.float32
+    assert torch.equal(mm(x.view(2, 3, K)), want.view(2, 3, N))
+    assert mm(x[0]).shape == (N,) and torch.equal(mm(x[0]), mm(x[:1])[0])
+    wide = torch.zeros(6, 2 * K, device=dev)
+    wide[:, :K] = x
+    assert torch.equal(mm(wide[:, :K]), want)
+    out = torch.empty(6, N, device=dev)
+    assert mm(x, out=out) is out and torch.equal(out, want)
+    out = torch.empty(3, 2, N, device=dev)
+    got = mm(x, out=out)
+    assert got.shape == (6, N) and got.data_ptr() == out.data_ptr() and torch.equal(got, want)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        assert ops.stream_ptr().value == side.cuda_stream
+        got = mm(x)
+    side.synchronize()
+    assert torch.equal(got, want) and torch.equal(mm(x, stream=torch.cuda.current_stream()), want)

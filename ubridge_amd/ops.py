@@ -27,9 +27,18 @@ _DT_NAME = {torch.float32: "f32", torch.float16: "f16", torch.bfloat16: "bf16"}
 _Q_NAME = {Q4_0: "q4_0", Q8_0: "q8_0", Q4_K: "q4_k"}
 
 
+# The current stream's handle without making a Stream object: 0.45 us where
+# torch.cuda.current_stream() takes 2.8 us of an 11.6 us QMatMul call, whose
+# launch itself is 3.5 us.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def stream_ptr(stream=None):
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return ctypes.c_void_p(s.cuda_stream)
+    if stream is not None:
+        return ctypes.c_void_p(stream.cuda_stream)
+    if _raw_stream is None:
+        return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    return ctypes.c_void_p(_raw_stream(torch.cuda.current_device()))
 
 
 def _ptr(t):
@@ -128,15 +137,18 @@ class QMatMul:
         _need_cuda(x)
         if x.dtype not in (torch.float32, torch.bfloat16):
             raise ValueError("QMatMul takes f32 or bf16 activations")
-        x2 = x.reshape(-1, self.K).contiguous()
+        # decode calls are as long as their host side: no view is made of an x
+        # or a result that already has the shape
+        flat = x.dim() == 2 and x.shape[1] == self.K and x.is_contiguous()
+        x2 = x if flat else x.reshape(-1, self.K).contiguous()
         M = x2.shape[0]
         if out is None:
             out = torch.empty(M, self.N, dtype=out_dtype, device=x.device)
         ws = self.workspace(M)
-        check(lib.ubridge_qmatmul(self.qtype, _ptr(self.w), _ptr(x2), _DT_CODE[x2.dtype],
-                                  _ptr(out), _DT_CODE[out.dtype], M, self.N, self.K, _ptr(ws),
-                                  ws.numel(), stream_ptr(stream)))
-        return out.reshape(*x.shape[:-1], self.N)
+        check(lib.ubridge_qmatmul(self.qtype, self.w.data_ptr(), x2.data_ptr(), _DT_CODE[x2.dtype],
+                                  out.data_ptr(), _DT_CODE[out.dtype], M, self.N, self.K,
+                                  ws.data_ptr(), ws.numel(), stream_ptr(stream)))
+        return out if flat and out.shape == (M, self.N) else out.reshape(*x.shape[:-1], self.N)
 
     __call__ = forward
 
