@@ -262,6 +262,32 @@ def test_gemv_ring_exact_activations(dev, qt, N, K):
 
 
 @pytest.mark.parametrize("qt", [ops.Q4_0, ops.Q8_0, ops.Q4_K])
+@pytest.mark.parametrize("M,K,N", [(5, 1024, 50), (6, 5120, 77), (7, 4096, 4112), (8, 14336, 40),
+                                   (8, 2048, 6145), (3, 9216, 33), (3, 1024, 16400), (5, 4096, 16400),
+                                   (8, 5120, 16385)])
+def test_gemv_ring_8_tokens(dev, qt, M, K, N):
+    # up to 8 tokens the ring GEMV multiplies two neighbouring blocks at once:
+    # every default variant (16, 32 and 112 rows a workgroup, and the any-K
+    # one that takes K = 5120 on narrow and wide matrices), partial row tiles,
+    # used and unused token slots.  Losslessly quantizable activations: exact
+    # products, so only the order of the f32 sums differs from the dense dot.
+    N = -(-N // 8) * 8 if qt == ops.Q8_0 else N  # payload alignment
+    g = np.random.default_rng(M * K + N)
+    x = g.integers(-120, 121, (M, K)).astype(np.float32)
+    if qt == ops.Q4_K:
+        x.reshape(M, -1, 256)[:, :, 3] = -128.0
+    else:
+        x.reshape(M, -1, 32)[:, :, 3] = 127.0
+    x *= 2.0 ** g.integers(-3, 4, (M, 1)).astype(np.float32)  # another scale per token
+    w, y = _run(dev, qt, N, K, x)
+    wd = oracle.dequant(qt, w, N * K, oracle.F32).reshape(N, K)
+    # per token: the bound is that of K f32 additions relative to the row
+    want = (torch.from_numpy(x).double() @ torch.from_numpy(wd).double().T).numpy()
+    for t in range(M):
+        assert rel_err(y[t], want[t]) < 1e-6
+
+
+@pytest.mark.parametrize("qt", [ops.Q4_0, ops.Q8_0, ops.Q4_K])
 def test_gemv_ring_bf16_in_out(dev, qt):
     N, K, M = 300, 3072, 12
     x = synth.make_activations(M, K, seed=12)

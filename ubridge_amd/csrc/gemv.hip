@@ -2151,7 +2151,21 @@ struct MmCfg {
   static constexpr int PW = (TI + NW - 1) / NW;           // per wavefront (at most)
 };
 
-template <int QT, int OT, int RWV, int KG, int SB, int D, int HK>
+//
+// T8 (at most 8 tokens): half of the 16 token slots would be padding, and so
+// half of the f32 (Q4_K: integer) scaling of the products, which is what the
+// kernel issues most of.  One v_mfma_i32_16x16x64_i8 takes two neighbouring
+// blocks of a row at once: slot t < 8 holds token t's codes of the first block
+// and zeros for the second, slot t + 8 token t's codes of the second and zeros
+// for the first (each lane's 16 k lie in one block, so a lane reads either
+// its token's row or the zero row of an unused slot), and the two slots' sums
+// are added at the end.  Same products, half the scaling, 16-byte instead of
+// 8-byte LDS reads.  Quantize + GEMV at 8 tokens in a graph, weights from HBM
+// (us, before / after; K x N): Q8_0 4096 x 28672 29.2 / 27.7, 4096 x 6144 12.2
+// / 11.8, 4096 x 4096 10.4 / 10.0, 14336 x 4096 18.6 / 18.1; Q4_0 21.2 / 17.8,
+// 10.5 / 9.2, 8.6 / 8.0, 15.1 / 13.9; Q4_K 19.2 / 18.5, 9.9 / 9.7, 9.1 / 9.0,
+// 15.2 / 15.1.  5 to 7 tokens: as 8.
+template <int QT, int OT, int RWV, int KG, int SB, int D, int HK, bool T8>
 __global__ void __launch_bounds__(64 * RWV * KG) k_gemv_mm(GemvArgs a) {
   using C = MmCfg<QT, RWV, KG, SB>;
   constexpr int NW = C::NW, RT = C::RT, PW = C::PW;
@@ -2277,8 +2291,11 @@ __global__ void __launch_bounds__(64 * RWV * KG) k_gemv_mm(GemvArgs a) {
   float acc[4] = {0.f, 0.f, 0.f, 0.f};
   f32x4 mn = {0.f, 0.f, 0.f, 0.f};
   const int wrow = rw * 16 + r;  // this lane's row (A operand / headers) within the tile
-  // Q4_0: the lane's nibble moved to the byte's high half (low nibbles for h < 2)
-  const uint32_t nsh = 4u - 4u * (uint32_t)(h >> 1);
+  // Q4_0: the lane's nibble moved to the byte's high half (low nibbles for h <
+  // 2; T8: for even h); Q4_K, T8: to the low half (low nibbles for h < 2)
+  const uint32_t nsh = QT == UB_Q4_K ? 4u * (uint32_t)(h >> 1)
+                                     : 4u - 4u * (uint32_t)(T8 ? h & 1 : h >> 1);
+  constexpr int tmask = T8 ? 7 : 15;  // token of slot r
 
   // Block headers of the whole tile (16 B per row and 256 elements), once:
   // row r's headers are contiguous in memory, so the tile's are one run.  In
@@ -2306,9 +2323,14 @@ __global__ void __launch_bounds__(64 * RWV * KG) k_gemv_mm(GemvArgs a) {
     const uint32_t sb = ring0 + (uint32_t)((st % D) * C::SU * 16);
     // fragment bases: lane (row / token r, k-group h) reads 8 bytes at +8h of
     // each 32-byte run, so every read below is base + a constant
-    uint32_t cbase = sb + (uint32_t)((C::oWC + (gw * RT + wrow) * C::CUP) * 16 +
-                                     (QT == UB_Q4_0 ? 8 * (h & 1) : 8 * h));
-    uint32_t abase = sb + (uint32_t)((C::oAC + (gw * 16 + r) * C::AUP) * 16 + 8 * h);
+    // (T8: 16 bytes at +16h of each 64-byte run; Q4_0 / Q4_K pairs of blocks
+    // are 32 code bytes)
+    constexpr bool kNib = QT != UB_Q8_0;
+    const int coff = !T8 ? (QT == UB_Q4_0 ? 8 * (h & 1) : 8 * h)
+                         : kNib ? 16 * (QT == UB_Q4_0 ? h >> 1 : h & 1) : 16 * h;
+    uint32_t cbase = sb + (uint32_t)((C::oWC + (gw * RT + wrow) * C::CUP) * 16 + coff);
+    const int aslot = !T8 || (h >> 1) == (r >> 3) ? r & tmask : r | 8;  // T8: r | 8 with r < 8, r: zero rows
+    uint32_t abase = sb + (uint32_t)((C::oAC + (gw * 16 + aslot) * C::AUP) * 16 + (T8 ? 16 * h : 8 * h));
     // opaque to the compiler: one base register per region and step, the
     // constant parts of every read folded into ds_read offsets (otherwise it
     // keeps one register per read and rebases each of them every step)
@@ -2325,15 +2347,23 @@ __global__ void __launch_bounds__(64 * RWV * KG) k_gemv_mm(GemvArgs a) {
 #pragma unroll
       for (int kbl = 0; kbl < SB; kbl++) {
         const float dAr = __uint_as_float(ub_lds_read4(dbase + kbl * 64 + 4 * r));  // token r
-        const uint4 dA4 = ub_lds_read16(dbase + kbl * 64 + 16 * h);  // tokens 4h..4h+3
+        const uint4 dA4 = ub_lds_read16(dbase + kbl * 64 + 16 * (T8 ? h & 1 : h));  // tokens 4h..4h+3
         // header of row wrow: d | dmin, then the 6-bit scales / mins of the 8
         // sub-blocks packed in 12 bytes (get_scale_min_k4)
         const uint4 hd = ub_lds_read16(hbase + 16 * kbl);
-        int sc[8];
+        int sc[8];  // T8: sc[p] is that of sub-block 2p + h / 2
+        if constexpr (T8) {
+          const uint32_t y = hd.y >> (8 * (h >> 1)), w = hd.w >> (8 * (h >> 1));
+          sc[0] = y & 63;
+          sc[1] = (y >> 16) & 63;
+          sc[2] = (w & 0xF) | (((y >> 6) & 3) << 4);
+          sc[3] = ((w >> 16) & 0xF) | (((y >> 22) & 3) << 4);
+        } else {
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-          sc[j] = (hd.y >> (8 * j)) & 63;
-          sc[4 + j] = ((hd.w >> (8 * j)) & 0xF) | (((hd.y >> (8 * j + 6)) & 3) << 4);
+          for (int j = 0; j < 4; j++) {
+            sc[j] = (hd.y >> (8 * j)) & 63;
+            sc[4 + j] = ((hd.w >> (8 * j)) & 0xF) | (((hd.y >> (8 * j + 6)) & 3) << 4);
+          }
         }
         const uint32_t zb = (hd.z >> (8 * h)) & 0xff, wb = (hd.w >> (8 * h)) & 0xff;
         const int m0 = zb & 63, m1 = (wb >> 4) | ((zb >> 6) << 4);  // mins of sub-blocks h, 4 + h
@@ -2345,6 +2375,18 @@ __global__ void __launch_bounds__(64 * RWV * KG) k_gemv_mm(GemvArgs a) {
         mn = __builtin_amdgcn_mfma_f32_16x16x4f32(dAr * (float)sa0, dmin * (float)m0, mn, 0, 0, 0);
         mn = __builtin_amdgcn_mfma_f32_16x16x4f32(dAr * (float)sa1, dmin * (float)m1, mn, 0, 0, 0);
         i32x4 I[8];
+        if constexpr (T8) {
+#pragma unroll
+          for (int p = 0; p < 4; p++) {
+            // code bytes 32p + 16 (h & 1).., low nibbles (sub-block 2p) for h
+            // < 2, high ones (2p + 1) for the rest
+            const uint4 raw = ub_lds_read16(cbase + kbl * 128 + 32 * p);
+            const uint4 av = ub_lds_read16(abase + kbl * 256 + 64 * p);
+            const i32x4 w = {(int)((raw.x >> nsh) & 0x0F0F0F0Fu), (int)((raw.y >> nsh) & 0x0F0F0F0Fu),
+                             (int)((raw.z >> nsh) & 0x0F0F0F0Fu), (int)((raw.w >> nsh) & 0x0F0F0F0Fu)};
+            I[p] = __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_bit_cast(i32x4, av), w, izero, 0, 0, 0);
+          }
+        } else
 #pragma unroll
         for (int p = 0; p < 4; p++) {
           // code bytes 32p + 8h.. (low nibbles: elements 64p + 8h.., high:
@@ -2362,7 +2404,7 @@ __global__ void __launch_bounds__(64 * RWV * KG) k_gemv_mm(GemvArgs a) {
         // sum_j sc_j dot_j in integer (|dot| < 2^16, sc < 2^6: 24-bit products)
         int T[4] = {0, 0, 0, 0};
 #pragma unroll
-        for (int j = 0; j < 8; j++) {
+        for (int j = 0; j < (T8 ? 4 : 8); j++) {
           T[0] += __mul24(sc[j], I[j][0]);
           T[1] += __mul24(sc[j], I[j][1]);
           T[2] += __mul24(sc[j], I[j][2]);
@@ -2374,7 +2416,8 @@ __global__ void __launch_bounds__(64 * RWV * KG) k_gemv_mm(GemvArgs a) {
         acc[3] += (dw * __uint_as_float(dA4.w)) * (float)T[3];
       }
     } else {
-      uint32_t dbase = sb + (uint32_t)((C::oAD + (gw * 16 + r) * 2 * SB) * 16);
+      // T8: token r % 8's scales, from block r / 8 of each pair
+      uint32_t dbase = sb + (uint32_t)((C::oAD + (gw * 16 + (r & tmask)) * 2 * SB) * 16) + (T8 ? 4 * (r >> 3) : 0);
       // headers of the lane's output rows 4h .. 4h + 3 (of the wave's 16)
       uint32_t obase = ub_lds_addr(hdr) + (uint32_t)(((rw * 16 + 4 * h) * (nbr + 1) + (st * KG + gw) * SB) * 16);
       const uint32_t rstr = (uint32_t)(nbr + 1) * 16;
@@ -2388,6 +2431,33 @@ __global__ void __launch_bounds__(64 * RWV * KG) k_gemv_mm(GemvArgs a) {
         for (int i = 0; i < 4; i++) hq[i] = ub_lds_read16(obase + (uint32_t)i * rstr + 16 * kbl);
         constexpr float dsc = QT == UB_Q4_0 ? 0.0625f : 1.0f;  // exact power of two
         i32x4 I[8];
+        if constexpr (T8) {
+#pragma unroll
+          for (int p = 0; p < 4; p++) {
+            uint4 w = ub_lds_read16(cbase + kbl * C::CB + (QT == UB_Q4_0 ? 32 : 64) * p);
+            if constexpr (QT == UB_Q4_0) {  // 16 (q - 8) as below; odd h: elements 16..31
+              w.x = ((w.x << nsh) & 0xF0F0F0F0u) ^ 0x80808080u;
+              w.y = ((w.y << nsh) & 0xF0F0F0F0u) ^ 0x80808080u;
+              w.z = ((w.z << nsh) & 0xF0F0F0F0u) ^ 0x80808080u;
+              w.w = ((w.w << nsh) & 0xF0F0F0F0u) ^ 0x80808080u;
+            }
+            const uint4 av = ub_lds_read16(abase + kbl * 256 + 64 * p);
+            I[p] = __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_bit_cast(i32x4, w),
+                                                         __builtin_bit_cast(i32x4, av), izero, 0, 0, 0);
+          }
+#pragma unroll
+          for (int p = 0; p < 4; p++) {
+            const float dA = __uint_as_float(ub_lds_read4(dbase + 4 * (kbl * 8 + 2 * p))) * dsc;
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+              const uint32_t hw = p == 0 ? hq[i].x : p == 1 ? hq[i].y : p == 2 ? hq[i].z : hq[i].w;
+              const _Float16 dw = __builtin_bit_cast(_Float16, (uint16_t)(hw >> (2 * (r & 8))));
+              const float t = __builtin_fmaf((float)dw, dA, 0.0f);
+              acc[i] += t * (float)I[p][i];
+            }
+          }
+          continue;
+        }
 #pragma unroll
         for (int j = 0; j < 8; j++) {
           // elements 32j + 8h ..: Q8_0 codes; Q4_0 bytes 8 (h & 1) .. of the
@@ -2438,6 +2508,11 @@ __global__ void __launch_bounds__(64 * RWV * KG) k_gemv_mm(GemvArgs a) {
     float v = red[t * RT + rr];
 #pragma unroll
     for (int g = 1; g < KG; g++) v += red[(g * 16 + t) * RT + rr];
+    if constexpr (T8) {
+      if (t >= 8) break;  // the second blocks' slots: added to token t - 8
+#pragma unroll
+      for (int g = 0; g < KG; g++) v += red[(g * 16 + t + 8) * RT + rr];
+    }
     if (t < M && row0 + rr < N) store_out<OT>(a.y, (size_t)t * N + row0 + rr, v);
   }
 }
@@ -2451,18 +2526,18 @@ constexpr int mm_lds() {
 
 constexpr int kMmMaxSb = 128;  // longest row the ring GEMV takes: 128 x 256 elements
 
-template <int QT, int OT, int RWV, int KG, int SB, int D, int HK>
+template <int QT, int OT, int RWV, int KG, int SB, int D, int HK, bool T8 = false>
 void launch_mm_t(const GemvArgs& a, hipStream_t s) {
   const int nbr = a.K / 256;
   constexpr bool fits = mm_lds<QT, RWV, KG, SB, D, HK>() <= 160 * 1024;
   if constexpr (fits) {
     if (nbr % (KG * SB) == 0 && nbr <= HK)
-      return k_gemv_mm<QT, OT, RWV, KG, SB, D, HK>
+      return k_gemv_mm<QT, OT, RWV, KG, SB, D, HK, T8>
           <<<ub_cdiv(a.N, 16 * RWV), 64 * RWV * KG, 0, s>>>(a);
   }
   // (variants that do not fit this block type's LDS, or this K) any K up to
   // kMmMaxSb super-blocks
-  k_gemv_mm<QT, OT, 1, 4, 1, 2, kMmMaxSb><<<ub_cdiv(a.N, 16), 256, 0, s>>>(a);
+  k_gemv_mm<QT, OT, 1, 4, 1, 2, kMmMaxSb, T8><<<ub_cdiv(a.N, 16), 256, 0, s>>>(a);
 }
 
 // Ring-GEMV variants <rows per workgroup / 16, K groups, super-blocks per
@@ -2474,10 +2549,19 @@ void launch_mm_t(const GemvArgs& a, hipStream_t s) {
 // while Q8_0's doubled stage no longer fits the LDS ring), below that
 // 32- or 16-row tiles with K split over 4 or 8 wavefront groups so that a
 // narrow matrix still spreads over the CUs (measured fastest on MI355X at the
-// configs[1] shapes).
+// Llama-3-8B widths).
 template <int QT, int OT>
 void launch_mm(int cfg, const GemvArgs& a, hipStream_t s) {
-  if (cfg <= 0) cfg = a.N >= 16384 ? (QT == UB_Q8_0 ? 1 : 13) : a.N > 4096 ? 5 : 7;
+  if (cfg <= 0) {
+    cfg = a.N >= 16384 ? (QT == UB_Q8_0 ? 1 : 13) : a.N > 4096 ? 5 : 7;
+    if (a.M <= 8) {  // the same shapes, two blocks per product (faster at every
+                     // size and format measured, see k_gemv_mm)
+      if (cfg == 1) return launch_mm_t<QT, OT, 7, 1, 1, 3, 16, true>(a, s);
+      if (cfg == 13) return launch_mm_t<QT, OT, 7, 2, 1, 2, 16, true>(a, s);
+      if (cfg == 5) return launch_mm_t<QT, OT, 2, 4, 1, 2, 56, true>(a, s);
+      return launch_mm_t<QT, OT, 1, 8, 1, 2, 56, true>(a, s);
+    }
+  }
   switch (cfg) {
     case 1: return launch_mm_t<QT, OT, 7, 1, 1, 3, 16>(a, s);
     case 2: return launch_mm_t<QT, OT, 7, 1, 2, 2, 16>(a, s);
