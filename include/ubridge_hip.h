@@ -103,7 +103,7 @@ int ubridge_workspace_stats(size_t* live_buffers, size_t* live_bytes, long* call
  * each owning 256x64, for M >= 2048; 6 = the slab route from 17 tokens; 7 =
  * no K split over workgroups in the pipelined GEMMs), "moe_gemm_path"
  * (grouped expert GEMM tile / load-ring variant,
- * 1..12), "gemv_mm" (the 3..16-token ring GEMV for Q4_0 / Q8_0 / Q4_K with K a
+ * 1..13), "gemv_mm" (the 3..16-token ring GEMV for Q4_0 / Q8_0 / Q4_K with K a
  * multiple of 1024: < 0 off, 1..22 a fixed tile / ring variant, taken from 3
  * tokens on), "gemv_persist" (one-launch quantize + GEMV: < 0 one workgroup
  * per row group, > 0 the persistent grid; 2 / 3 force the rolling prefetch

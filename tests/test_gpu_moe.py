@@ -244,6 +244,67 @@ def test_moe_tile_kernel(dev, moe_path, path, K, N, bs, q8, mrw, bias, emap, dty
     assert bool(((got - want).abs() <= ulp * want.abs() + 1e-4 * rms).all())
 
 
+@pytest.mark.parametrize("K,N,bs,q8,mrw,bias,emap,dtype", [
+    (128, 8, 32, True, 0, False, False, torch.bfloat16),     # one wavefront's K, one column block's edge
+    (768, 264, 32, True, 1, True, True, torch.bfloat16),     # idle wavefronts, partial block, -1 and shared experts
+    (1024, 72, 16, True, 1, False, True, torch.float16),     # two blocks per tile
+    (1152, 200, 32, True, 0, True, False, torch.float16),    # a second K step for one wavefront
+    (2048, 136, 4, True, 0, False, True, torch.bfloat16),
+    (1152, 72, 32, False, 0, True, False, torch.bfloat16),  # 16-bit weights
+    (2048, 136, 1, False, 0, False, True, torch.float16),
+    (1280, 264, 16, False, 1, True, True, torch.bfloat16)])
+def test_moe_stream_kernel(dev, moe_path, K, N, bs, q8, mrw, bias, emap, dtype):
+    # experts with 0, 1, 15 .. 17, 31 .. 33 and 70 rows, against f64, as above;
+    # and the gated form against silu_and_mul of the plain one
+    rows = [0, 1, 15, 16, 17, 0, 31, 32, 33, 70, 2, 1]
+    E, k = len(rows), 2
+    g = torch.Generator().manual_seed(K + N)
+    flat = torch.cat([torch.full((n,), e) for e, n in enumerate(rows)])
+    flat = flat[torch.randperm(flat.numel(), generator=g)]
+    T = flat.numel() // k
+    ids = flat[:T * k].view(T, k).int().to(dev)
+    em = None
+    if emap:  # neighbours 2 and 3 share an expert's weights, 6 and 9 are elsewhere
+        em = torch.arange(E, dtype=torch.int32)
+        em[3], em[6], em[9] = 2, -1, -1
+        em = em.to(dev)
+    s, e, n = moe.moe_align_block_size(ids, E, bs, expert_map=em)
+    A = torch.randn(T * k if mrw else T, K, generator=g).to(dtype).to(dev)
+    if q8:
+        B = torch.randint(-128, 128, (E, N, K), generator=g, dtype=torch.int8).to(dev)
+        Bs = (torch.rand(E, N, generator=g) * 0.01 + 0.001).to(dtype).to(dev)
+        Bf = B.double() * Bs.double()[:, :, None]
+    else:
+        B, Bs = torch.randn(E, N, K, generator=g).to(dtype).to(dev), None
+        Bf = B.double()
+    bv = torch.randn(E, N, generator=g).to(dtype).to(dev) if bias else None
+    tw = torch.rand(T * k, generator=g).to(dev)
+    C = torch.full((T * k + 1, N), 3.0, dtype=dtype, device=dev)
+    moe_path(13)
+    moe.invoke_fused_moe(A, B, C[:T * k], tw if mrw else None, s, e, n, k, bs, mrw, B_scale=Bs,
+                         bias=bv)
+    ex = ids.flatten().long() if em is None else em.long()[ids.flatten().long()]
+    here = ex >= 0
+    a = A.double() if mrw else A.double().repeat_interleave(k, 0)
+    want = torch.zeros(T * k, N, dtype=torch.float64, device=dev)
+    for q in range(E):
+        r = ex == q
+        want[r] = a[r] @ Bf[q].T.contiguous() + (bv[q].double() if bias else 0.0)
+    if mrw:
+        want *= tw.double()[:, None] * here[:, None]
+    got = C[:T * k].double()
+    assert bool((got[~here] == 0).all()) and bool((C[T * k] == 3.0).all())
+    # one rounding to T of an f32 sum (error far below it)
+    ulp = 2.0**-8 if dtype == torch.bfloat16 else 2.0**-10
+    rms = want[here].square().mean().sqrt()
+    assert bool(((got - want).abs() <= ulp * want.abs() + 1e-4 * rms).all())
+    if not mrw:
+        act = torch.full((T * k + 1, N // 2), 7.0, dtype=dtype, device=dev)
+        moe.fused_moe_gate_up_silu(A, B, Bs, s, e, n, k, bs, bias=bv, out=act[:T * k], topk_ids_size=T * k)
+        assert torch.equal(act[:T * k].view(torch.int16), moe.silu_and_mul(C[:T * k]).view(torch.int16))
+        assert bool((act[T * k] == 7.0).all())
+
+
 def test_moe_tile_windows(dev, moe_path):
     # more tiles than the list in LDS holds (512): 700 experts of one block
     # and 5 large ones; the same bits as the 32-row kernel
@@ -261,6 +322,32 @@ def test_moe_tile_windows(dev, moe_path):
         out.append(moe.invoke_fused_moe(A, B, C, None, s, e, n, k, 32, False))
     assert torch.equal(out[0].view(torch.int16), out[1].view(torch.int16))
     assert torch.equal(out[0].view(torch.int16), out[2].view(torch.int16))
+
+
+def test_moe_stream_rule_and_bad_expert(dev, moe_path):
+    # the automatic choice takes the stream for few blocks and gives its bits;
+    # an expert id past E leaves its rows alone and sets the device flag
+    T, k, E, K, N = 7, 2, 8, 1024, 392
+    g = torch.Generator().manual_seed(3)
+    ids = torch.randint(0, E, (T, k), generator=g, dtype=torch.int32).to(dev)
+    s, e, n = moe.moe_align_block_size(ids, E, 32)
+    A = torch.randn(T, K, generator=g).bfloat16().to(dev)
+    B = torch.randint(-128, 128, (E, N, K), generator=g, dtype=torch.int8).to(dev)
+    Bs = (torch.rand(E, N, generator=g) * 0.01).bfloat16().to(dev)
+    C = [torch.zeros(T * k, N, dtype=torch.bfloat16, device=dev) for _ in range(3)]
+    for path, c in zip((0, 13, 1), C):
+        moe_path(path)
+        moe.invoke_fused_moe(A, B, c, None, s, e, n, k, 32, False, B_scale=Bs)
+    assert torch.equal(C[0], C[1]) and rel_err(C[0].double().cpu().numpy(), C[2].double().cpu().numpy()) < 4e-3
+    bad = int(e[0])
+    e[0] = E + 1
+    c = torch.full((T * k, N), 3.0, dtype=torch.bfloat16, device=dev)
+    moe_path(0)
+    moe.invoke_fused_moe(A, B, c, None, s, e, n, k, 32, False, B_scale=Bs)
+    with pytest.raises(_lib.UbridgeError):
+        moe.device_error()
+    here = ids.flatten() == bad
+    assert bool((c[here] == 3.0).all()) and torch.equal(c[~here], C[0][~here])
 
 
 def test_moe_tile_bad_expert_flagged(dev, moe_path):

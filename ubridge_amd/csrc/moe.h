@@ -27,3 +27,7 @@ struct MoeArgs {
 // these sizes, 0 where k_moe_gemm is faster.
 bool ub_moe_tile(const MoeArgs& a, int rows, int dt, bool q8, int* err, hipStream_t s);
 int ub_moe_tile_rows(const MoeArgs& a, bool q8);
+
+// The same for decode batches whose blocks leave CUs idle (moe_stream.hip).
+bool ub_moe_stream(const MoeArgs& a, int dt, bool q8, int* err, hipStream_t s);
+bool ub_moe_stream_pays(const MoeArgs& a, bool q8);

@@ -837,7 +837,8 @@ __global__ void __launch_bounds__(64 * NWV) k_moe_gemm(MoeArgs a) {
 // 4: 256 columns, BK 128, 3 stages (int8 only); 5: 128 columns, BK 64,
 // 4 stages; 6 / 7: 64 columns, BK 64, 4 / 6 stages; 8: 128 columns, BK 64,
 // 3 stages; 9: 64 columns, BK 128, 3 stages; 10 / 11 / 12: the 128-, 64- and
-// (int8) 32-row tiles of moe_tile.hip.  Automatic (0): those where
+// (int8) 32-row tiles of moe_tile.hip; 13: the stream of moe_stream.hip.
+// Automatic (0): the last where ub_moe_stream_pays, the tiles where
 // ub_moe_tile_rows says so, else 1 while its workgroups (about one block per
 // expert in use and 32 slots, times the column blocks) fit the CUs at once, two
 // per CU, and 8 (half the LDS, four per CU) beyond: 128 experts, int8 gate/up +
@@ -916,6 +917,8 @@ int moe_gemm(const char* nm, int dt, bool q8, void* C, const void* A, const void
   const int max_blocks = (tis + E * (bs - 1)) / bs;
   hipStream_t s = ub_stream(stream);
   const int path = ub_tune(UB_TUNE_MOE_GEMM_PATH);
+  if ((path == 13 || (path == 0 && ub_moe_stream_pays(a, q8))) && ub_moe_stream(a, dt, q8, error_flag(), s))
+    return ub_check_launch(nm);
   const int rows = path == 0 ? ub_moe_tile_rows(a, q8) : path == 10 ? 128 : path == 11 ? 64 : path == 12 && q8 ? 32 : 0;
   if (rows && ub_moe_tile(a, rows, dt, q8, error_flag(), s)) return ub_check_launch(nm);
   if (dt == UB_BF16) {
