@@ -388,6 +388,23 @@ def test_fused_moe_expert_minus_one_zeroes(dev):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("E,k,bs,norm", [(1, 1, 32, 1), (64, 6, 32, 0), (65, 64, 16, 1), (128, 8, 32, 1),
+                                         (129, 16, 4, 0), (256, 16, 32, 1), (256, 17, 32, 0), (257, 8, 64, 1)])
+@pytest.mark.parametrize("T", [1, 3, 8, 9])
+def test_moe_route_one_launch_bits(dev, dtype, E, k, bs, norm, T):
+    # routing of up to 8 tokens in one launch, on both sides of its limits
+    # (8 tokens, 128 / 256 experts, 16 picks), ties included, against the two
+    # operators bit for bit
+    g = torch.Generator().manual_seed(T * E + k)
+    logits = (torch.randint(-9, 10, (T, E), generator=g) / 4).to(dtype).to(dev)
+    w, wf, ids, s, e, n = moe.moe_route(logits, k, E, bs, bool(norm))
+    w2, ids2 = moe.topk_softmax(logits, k, bool(norm))
+    s2, e2, n2 = moe.moe_align_block_size(ids2, E, bs)
+    assert torch.equal(w, w2) and torch.equal(wf, w2.float()) and torch.equal(ids, ids2)
+    assert torch.equal(s, s2) and torch.equal(e, e2) and torch.equal(n, n2)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("T,E,k,bs,norm", [(256, 128, 8, 32, 1), (37, 60, 3, 16, 0), (5, 200, 6, 4, 1),
                                            (600, 64, 8, 64, 1), (1, 8, 2, 32, 0)])
 def test_moe_route_matches_separate_ops(dev, dtype, T, E, k, bs, norm):

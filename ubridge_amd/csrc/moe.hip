@@ -17,6 +17,7 @@
 #include "registry.h"
 
 #include <algorithm>
+#include <type_traits>
 #include <atomic>
 
 namespace {
@@ -499,6 +500,22 @@ size_t align_small_lds(int n, int E) {
   const int nc = (n + 63) / 64;
   const int G = std::max(1, std::min(nc, kRouteThreads / E));
   return sizeof(int) * ((size_t)nc * E + (size_t)G * E + E + 2);
+}
+
+// Top-k and align of at most kRouteTokens tokens in one workgroup, a wavefront
+// (E <= 128) or a 16-lane group per token: both are chains of latencies that a
+// second launch only lengthens.  The ids meet in global memory at the barrier.
+constexpr int kRouteTokens = 8;
+template <int DT, int G, int NPL>
+__global__ void __launch_bounds__(kRouteThreads) k_moe_route_small(
+    const void* __restrict__ in, void* __restrict__ out, int* ids, float* __restrict__ wf32,
+    int* __restrict__ sorted, int* __restrict__ experts, int* __restrict__ ntpp, int T, int E,
+    int k, int norm, int bs) {
+  extern __shared__ int sh[];
+  topk_tokens<DT, G, NPL>(in, out, ids, wf32, nullptr, threadIdx.x / G, kRouteThreads / G, T, E, k,
+                          norm, threadIdx.x % G);
+  __syncthreads();
+  align_small_body(ids, sh, sorted, experts, ntpp, T * k, E, bs);
 }
 
 bool align_small_ok(int n, int E) { return n > 0 && n <= kRouteMaxN && align_small_lds(n, E) <= 96 * 1024; }
@@ -1077,10 +1094,15 @@ UB_API void topk_softmax_bf16(const void* in, void* out, int* idx, int T, int E,
 
 // Routing for the grouped GEMM in one call: topk_softmax (T weights and ids,
 // plus their f32 values for the GEMM's routed-weight operand) and
-// moe_align_block_size, as two launches: the top-k over the whole GPU (one
-// token per lane group) and the align in one workgroup.  (Both in one
-// 1024-thread workgroup measured 2.5x slower at 256 tokens x 128 experts:
-// the top-k needs the GPU's parallelism more than a launch is worth.)
+// moe_align_block_size.  Up to 8 tokens and 256 experts in one launch
+// (k_moe_route_small); beyond as two: the top-k over
+// the whole GPU (one token per lane group) and the align.  Both in one
+// 1024-thread workgroup at 256 tokens x 128 experts measured 2.5x slower: the
+// top-k needs the GPU's parallelism more than a launch is worth.  us, two
+// launches / one: 128 experts top-8, 1 token 7.8 / 6.7, 8 tokens 8.2 / 7.4, 16
+// tokens 8.3 / 9.4 (four wavefronts of a SIMD in step); 64 experts top-6 6.6 /
+// 5.4, 6.9 / 5.9, 7.2 / 7.4; 8 experts top-2 5.4 / 4.3, 5.6 / 4.5, 5.8 / 5.3;
+// 256 experts top-8 12.4 / 11.4, 12.3 / 11.2, 12.7 / 11.7.
 static int moe_align_launch(int* sorted_ids, int* experts_ids, int* num_tokens_post_pad,
                             const int* topk_ids, const int* real_token_num,
                             const int* expert_map, int num_experts, int block_size,
@@ -1096,6 +1118,25 @@ UB_API int ubridge_moe_route(const void* logits, int dtype, void* topk_w, float*
   UB_REQUIRE(dtype == UB_F32 || dtype == UB_F16 || dtype == UB_BF16, "%s: dtype %d", nm, dtype);
   UB_REQUIRE(logits && topk_w && topk_ids && sorted_ids && experts_ids && num_tokens_post_pad,
              "%s: null pointer", nm);
+  if (T > 0 && T <= kRouteTokens && E <= 256 && (E <= 128 || k <= 16) && align_small_ok(T * k, E)) {
+    const size_t lds = align_small_lds(T * k, E);
+    hipStream_t s = ub_stream(stream);
+    auto go = [&](auto kern) {  // lane groups and registers as topk_softmax_launch chooses them
+      (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+      kern<<<1, kRouteThreads, lds, s>>>(logits, topk_w, topk_ids, topk_w_f32, sorted_ids, experts_ids,
+                                         num_tokens_post_pad, T, E, k, renormalize, block_size);
+    };
+    auto pick = [&](auto dtc) {
+      constexpr int DT = decltype(dtc)::value;
+      if (E <= 64) go(k_moe_route_small<DT, 64, 1>);
+      else if (E <= 128) go(k_moe_route_small<DT, 64, 2>);
+      else go(k_moe_route_small<DT, 16, 16>);
+    };
+    if (dtype == UB_F32) pick(std::integral_constant<int, UB_F32>{});
+    else if (dtype == UB_F16) pick(std::integral_constant<int, UB_F16>{});
+    else pick(std::integral_constant<int, UB_BF16>{});
+    return ub_check_launch(nm);
+  }
   int e = dtype == UB_F32   ? topk_softmax_launch<UB_F32>(logits, topk_w, topk_ids, T, E, k,
                                                          renormalize, stream, nm, topk_w_f32)
           : dtype == UB_F16 ? topk_softmax_launch<UB_F16>(logits, topk_w, topk_ids, T, E, k,
