@@ -305,6 +305,46 @@ def test_moe_stream_kernel(dev, moe_path, K, N, bs, q8, mrw, bias, emap, dtype):
         assert bool((act[T * k] == 7.0).all())
 
 
+@pytest.mark.parametrize("path", [10, 11, 12])  # tiles of 128, 64, 32 rows
+@pytest.mark.parametrize("K,N,bs,mrw,bias,emap,dtype", [
+    (64, 8, 32, 0, False, False, torch.bfloat16), (128, 264, 32, 1, True, True, torch.bfloat16),
+    (192, 520, 16, 0, True, False, torch.float16), (768, 256, 32, 1, False, False, torch.bfloat16),
+    (2048, 72, 4, 0, False, True, torch.float16)])
+def test_moe_tile_int8_bits(dev, moe_path, path, K, N, bs, mrw, bias, emap, dtype):
+    # int8 experts: the tiles give the bits of the 32-row kernel at every row
+    # count, so that what a token gets does not change with the batch it is in
+    # (1024 rows of one expert more: tiles that follow one another on a
+    # workgroup); also the gated form
+    rows = [0, 1, 31, 32, 33, 0, 64, 65, 95, 96, 97, 127, 128, 129, 1324, 2]
+    E, k = len(rows), 2
+    g = torch.Generator().manual_seed(K + N)
+    flat = torch.cat([torch.full((n,), e) for e, n in enumerate(rows)])
+    flat = flat[torch.randperm(flat.numel(), generator=g)]
+    T = flat.numel() // k
+    ids = flat[:T * k].view(T, k).int().to(dev)
+    em = None
+    if emap:
+        em = torch.arange(E, dtype=torch.int32)
+        em[3], em[6] = 2, -1
+        em = em.to(dev)
+    s, e, n = moe.moe_align_block_size(ids, E, bs, expert_map=em)
+    A = (torch.randn(T * k if mrw else T, K, generator=g) * 3).to(dtype).to(dev)
+    B = torch.randint(-128, 128, (E, N, K), generator=g, dtype=torch.int8).to(dev)
+    Bs = (torch.rand(E, N, generator=g) * 0.01 + 0.001).to(dtype).to(dev)
+    bv = torch.randn(E, N, generator=g).to(dtype).to(dev) if bias else None
+    tw = torch.rand(T * k, generator=g).to(dev) if mrw else None
+    out = []
+    for p in (1, path):
+        moe_path(p)
+        C = torch.full((T * k, N), 3.0, dtype=dtype, device=dev)
+        out.append([moe.invoke_fused_moe(A, B, C, tw, s, e, n, k, bs, mrw, B_scale=Bs, bias=bv)])
+        if not mrw:
+            out[-1].append(moe.fused_moe_gate_up_silu(A, B, Bs, s, e, n, k, bs, bias=bv,
+                                                      out=torch.full_like(C[:, :N // 2], 3.0)))
+    for a, b in zip(*out):
+        assert torch.equal(a.view(torch.int16), b.view(torch.int16))
+
+
 def test_moe_tile_windows(dev, moe_path):
     # more tiles than the list in LDS holds (512): 700 experts of one block
     # and 5 large ones; the same bits as the 32-row kernel

@@ -13,7 +13,7 @@
 // ubridge_device_error() reads after synchronizing the stream.
 #include "common.h"
 #include "lds_dma.h"
-#include "moe.h"
+#include "moe_dev.h"
 #include "registry.h"
 
 #include <algorithm>
@@ -30,11 +30,6 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 constexpr uint32_t kOOB = 0x80000000u;
 
-template <int DT>
-__device__ __forceinline__ float tof(uint16_t b) {
-  if constexpr (DT == UB_BF16) return ub_bf16_to_f32(b);
-  else return ub_f16_to_f32(b);
-}
 template <int DT>
 __device__ __forceinline__ uint16_t fromf(float v) {
   if constexpr (DT == UB_BF16) return __builtin_bit_cast(unsigned short, (__bf16)v);
@@ -555,49 +550,6 @@ __device__ __forceinline__ f32x16 mfma(const uint4& a, const uint4& b, const f32
   else
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a),
                                                   __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
-}
-
-// 8 int8 (two dwords) -> 8 T holding q + 128 (exact: 0..255 fit T's
-// significand); the caller subtracts 128 * (sum of the A row) after the
-// dot.  1.75 VALU ops per value: one xor per 4, a byte convert each, one
-// pack per 2.
-template <int DT>
-__device__ __forceinline__ uint4 i8x8_to_t_off(uint32_t lo, uint32_t hi) {
-  typedef unsigned char u8x4 __attribute__((ext_vector_type(4)));
-  typedef float f32x2 __attribute__((ext_vector_type(2)));
-  const u8x4 L = __builtin_bit_cast(u8x4, lo ^ 0x80808080u), H = __builtin_bit_cast(u8x4, hi ^ 0x80808080u);
-  uint32_t o[4];
-#pragma unroll
-  for (int i = 0; i < 4; i++) {
-    const u8x4& V = i < 2 ? L : H;
-    const f32x2 f = {(float)V[2 * (i & 1)], (float)V[2 * (i & 1) + 1]};
-    if constexpr (DT == UB_BF16) {
-      typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-      o[i] = __builtin_bit_cast(uint32_t, __builtin_convertvector(f, bf16x2));
-    } else {
-      typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
-      o[i] = __builtin_bit_cast(uint32_t, __builtin_convertvector(f, f16x2));
-    }
-  }
-  return make_uint4(o[0], o[1], o[2], o[3]);
-}
-// acc + the sum of the 8 T values of an MFMA fragment (f32, by v_dot2)
-template <int DT>
-__device__ __forceinline__ float frag_sum(const uint4& a, float acc) {
-  const uint32_t w[4] = {a.x, a.y, a.z, a.w};
-#pragma unroll
-  for (int i = 0; i < 4; i++) {
-    if constexpr (DT == UB_BF16) {
-      typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-      const bf16x2 one = {(__bf16)1.0f, (__bf16)1.0f};
-      acc = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, w[i]), one, acc, false);
-    } else {
-      typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
-      const f16x2 one = {(_Float16)1.0f, (_Float16)1.0f};
-      acc = __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2, w[i]), one, acc, false);
-    }
-  }
-  return acc;
 }
 
 // s_waitcnt vmcnt(n) for a wave-uniform runtime n (clamped to 15: waiting

@@ -1,5 +1,5 @@
-// moe_dev.h -- device code shared by the grouped expert GEMMs on tiles of
-// sorted blocks (moe_tile.hip, moe_stream.hip).
+// moe_dev.h -- device code shared by the grouped expert GEMMs (moe.hip,
+// moe_tile.hip, moe_stream.hip).
 #pragma once
 #include "moe.h"
 
@@ -52,6 +52,53 @@ __device__ __forceinline__ uint4 i8x8_to_t(uint32_t lo, uint32_t hi) {
       o[i] = __builtin_bit_cast(uint32_t, (f16x2)(__builtin_bit_cast(f16x2, p[i]) - off));
   }
   return make_uint4(o[0], o[1], o[2], o[3]);
+}
+
+// 8 int8 (two dwords) -> 8 T holding q + 128 (exact: 0..255 fit T's
+// significand); the caller subtracts 128 * (sum of the A row) after the
+// dot.  bf16: 1.75 VALU ops per value: one xor per 4, a byte convert each,
+// one pack per 2.
+template <int DT>
+__device__ __forceinline__ uint4 i8x8_to_t_off(uint32_t lo, uint32_t hi) {
+  const uint32_t l = lo ^ 0x80808080u, h = hi ^ 0x80808080u;
+  uint32_t o[4];
+  if constexpr (DT == UB_BF16) {
+    typedef unsigned char u8x4 __attribute__((ext_vector_type(4)));
+    const u8x4 L = __builtin_bit_cast(u8x4, l), H = __builtin_bit_cast(u8x4, h);
+    o[0] = pack2<DT>((float)L[0], (float)L[1]);
+    o[1] = pack2<DT>((float)L[2], (float)L[3]);
+    o[2] = pack2<DT>((float)H[0], (float)H[1]);
+    o[3] = pack2<DT>((float)H[2], (float)H[3]);
+  } else {
+    // the byte q + 128 under 0x64 is the f16 1024 + (q + 128)
+    typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+    const f16x2 off = {(_Float16)1024.0f, (_Float16)1024.0f};
+    const uint32_t m = 0x64646464u;
+    const uint32_t p[4] = {__builtin_amdgcn_perm(m, l, 0x04010400u), __builtin_amdgcn_perm(m, l, 0x04030402u),
+                           __builtin_amdgcn_perm(m, h, 0x04010400u), __builtin_amdgcn_perm(m, h, 0x04030402u)};
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+      o[i] = __builtin_bit_cast(uint32_t, (f16x2)(__builtin_bit_cast(f16x2, p[i]) - off));
+  }
+  return make_uint4(o[0], o[1], o[2], o[3]);
+}
+// acc + the sum of the 8 T values of an MFMA fragment (f32, by v_dot2)
+template <int DT>
+__device__ __forceinline__ float frag_sum(const uint4& a, float acc) {
+  const uint32_t w[4] = {a.x, a.y, a.z, a.w};
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    if constexpr (DT == UB_BF16) {
+      typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+      const bf16x2 one = {(__bf16)1.0f, (__bf16)1.0f};
+      acc = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, w[i]), one, acc, false);
+    } else {
+      typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+      const f16x2 one = {(_Float16)1.0f, (_Float16)1.0f};
+      acc = __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2, w[i]), one, acc, false);
+    }
+  }
+  return acc;
 }
 
 // Cuts the sorted blocks into tiles (consecutive blocks of one expert, G at

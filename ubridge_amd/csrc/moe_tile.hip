@@ -31,16 +31,27 @@
 //    spilled), the one barrier per K-step sits before the last substep.  The
 //    next pair's rows are fetched during the K loop and its first stages are
 //    in flight during the epilogue.
-//  * int8 is exact in T; scale, bias and routed weight are applied to the f32
-//    sums as in k_moe_gemm.
+//  * int8 enters as q + 128 (exact in T) and 128 x the sum of the A row is
+//    subtracted from the f32 sums, in k_moe_gemm's order of additions: an
+//    output has the same bits from every tile height and from that kernel,
+//    whatever batch its token is in.  A wavefront sums the rows of one row
+//    tile only (its first: the wavefronts start at different row tiles) and
+//    the sums meet in LDS.  All four wavefronts summing all rows took 564 us
+//    for the whole 4096-token layer below, this way 472, the signed weights
+//    with nothing to subtract 472 (but other bits than k_moe_gemm's: 3e-4 of
+//    relative 2-norm in a bf16 layer).
+//  * scale, bias and routed weight are applied to the f32 sums as in
+//    k_moe_gemm.
 //
-// MI355X, 128 experts of 2048 -> 2 x 768 -> 2048, top-8, us (k_moe_gemm /
-// 128-row tiles), int8 at 1024 tokens: gate/up 194 / 125, down 100 / 75; at 4096: 587 /
-// 271, 301 / 165 (760 / 626 TFLOP/s); bf16 at 1024: 263 / 212, 205 / 110; at
-// 4096: 751 / 348, 704 / 198.  At 4096 int8 tokens the gate/up launch without
-// its epilogue takes 25 us less, with every load an L2 hit 34 us less, without
-// the int8 conversion 26 us less and without all three 200 us: MFMA issue
-// and LDS reads in step with a barrier per K-step hold most of it.
+// MI355X, 128 experts of 2048 -> 2 x 768 -> 2048, top-8, us in a graph of
+// launches with weights from HBM (k_moe_gemm / 64-row / 128-row tiles), int8 at
+// 1024 tokens: gate/up 203 / 124 / 137, down 132 / 77 / 81; at 4096: 582 / -
+// / 281, 423 / - / 166 (735 / 620 TFLOP/s); bf16 (k_moe_gemm / 128-row tiles)
+// at 1024: 263 / 212, 205 / 110; at 4096: 751 / 348, 704 / 198.  At 4096 int8
+// tokens the gate/up launch without its epilogue took 25 us less, with every
+// load an L2 hit 34 us less, without the int8 conversion (of the signed
+// weights) 26 us less and without all three 200 us: MFMA issue and LDS reads in
+// step with a barrier per K-step hold most of it.
 #include "lds_dma.h"
 #include "moe_dev.h"
 
@@ -87,6 +98,7 @@ k_moe_tile(MoeArgs a, int* err) {
   __shared__ __attribute__((aligned(16))) int srow[2][kTM];   // the tile's slots, -1: padding
   __shared__ __attribute__((aligned(16))) float stw[2][kTM];  // their routed weights
   __shared__ float ssc[2][Q8 ? BN : 1], sbv[2][BN];           // scale / bias of the weight rows
+  __shared__ __attribute__((aligned(16))) float srsum[2][Q8 ? kTM : 4];  // int8: sums of the A rows
   __shared__ int wsum[2][NWV];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -237,9 +249,20 @@ k_moe_tile(MoeArgs a, int* err) {
 #pragma unroll
           for (int r = 0; r < 16; r++) acc[i][j][r] = 0.f;
       uint4 af[2][TM], bf[2][2], bw[2];
+      // int8: each wavefront starts with another row tile (its i-th is tile
+      // (i + wave) % TM), whose rows it sums; 16-bit: in order.  Opaque, or an
+      // address per tile and substep would be kept and spilled (4096 tokens:
+      // 489 us a layer, 472 this way)
+      uint32_t tile_of[TM];
+#pragma unroll
+      for (int i = 0; i < TM; i++) {
+        tile_of[i] = Q8 ? (uint32_t)(i + wave) % TM : i;
+        if constexpr (Q8) asm("" : "+s"(tile_of[i]));
+      }
+      float rsum = 0.f;  // sum of the lane's row of tile_of[0] over its k half
       auto read_a = [&](uint32_t st, int s) {
 #pragma unroll
-        for (int i = 0; i < TM; i++) af[s & 1][i] = ub_lds_read16(st + aoff[s] + 32 * RA * i);
+        for (int i = 0; i < TM; i++) af[s & 1][i] = ub_lds_read16(st + aoff[s] + 32 * RA * tile_of[i]);
       };
       auto read_b = [&](uint32_t st, int s, uint4 (&to)[2]) {
 #pragma unroll
@@ -270,10 +293,16 @@ k_moe_tile(MoeArgs a, int* err) {
 #pragma unroll
           for (int j = 0; j < 2; j++) {
             const uint4& w = bw[j];
-            bf[s & 1][j] = (s & 1) ? i8x8_to_t<DT>(w.z, w.w) : i8x8_to_t<DT>(w.x, w.y);
+            bf[s & 1][j] = (s & 1) ? i8x8_to_t_off<DT>(w.z, w.w) : i8x8_to_t_off<DT>(w.x, w.y);
             // pinned here: the converts would otherwise sink to the MFMAs
             asm volatile("" : "+v"(bf[s & 1][j].x), "+v"(bf[s & 1][j].y), "+v"(bf[s & 1][j].z), "+v"(bf[s & 1][j].w));
           }
+        };
+        // the fragments' sum, pinned here as well (the sums would otherwise
+        // sink to the end of the K-step and keep the fragments)
+        auto add_rows = [&](int s) {
+          rsum = frag_sum<DT>(af[s & 1][0], rsum);
+          asm volatile("" : "+v"(rsum));
         };
         // one substep's instructions interleaved: MFMA, LDS read, VALU
         auto sched = [&](auto nreads) {
@@ -297,21 +326,25 @@ k_moe_tile(MoeArgs a, int* err) {
             const uint32_t cur = sbase + u * STB, nxt = sbase + (u + 1) % NS * STB;
             read_a(cur, 1);
             mfmas(0);
+            add_rows(0);
             widen(1);
             sched(std::integral_constant<int, TM>{});
             read_b(cur, 2, bw);
             read_a(cur, 2);
             mfmas(1);
+            add_rows(1);
             widen(2);
             sched(std::integral_constant<int, TM + 2>{});
             read_a(cur, 3);
             mfmas(2);
+            add_rows(2);
             widen(3);
             sched(std::integral_constant<int, TM>{});
             turn(kt, cur);
             read_b(nxt, 0, bw);
             read_a(nxt, 0);
             mfmas(3);
+            add_rows(3);
             widen(0);
             sched(std::integral_constant<int, TM + 2>{});
           }
@@ -343,9 +376,13 @@ k_moe_tile(MoeArgs a, int* err) {
             sched();
           }
       }
+      if constexpr (Q8) {  // read back behind the barrier of next()
+        rsum += __shfl_xor(rsum, 32);
+        if (wave < TM && kh == 0) srsum[buf][32 * wave + l32] = rsum;
+      }
       next();
-      // epilogue: register r of tile (i, j): token row 32 i + 8 (r / 4) + 4 kh
-      // + r % 4, tile row wave 64 + 32 j + l32 of the weight
+      // epilogue: register r of tile (i, j): token row 32 tile_of[i] + 8 (r /
+      // 4) + 4 kh + r % 4, tile row wave 64 + 32 j + l32 of the weight
       uint16_t* C = (uint16_t*)a.C;
       const bool bias = a.bias != nullptr, mrw = a.mrw != 0;
       float sc[2], bv[2];
@@ -360,18 +397,20 @@ k_moe_tile(MoeArgs a, int* err) {
         for (int i = 0; i < TM; i++)
 #pragma unroll
           for (int g = 0; g < 4; g++) {
-            const int r0 = 32 * i + 8 * g + 4 * kh;
+            const int r0 = 32 * tile_of[i] + 8 * g + 4 * kh;
             const int4 s4 = *(const int4*)&srow[buf][r0];
             const float4 t4 = *(const float4*)&stw[buf][r0];
+            const float4 q4 = Q8 ? *(const float4*)&srsum[buf][r0] : make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
             for (int x = 0; x < 4; x++) {
               const int s = x == 0 ? s4.x : x == 1 ? s4.y : x == 2 ? s4.z : s4.w;
               const float tw = x == 0 ? t4.x : x == 1 ? t4.y : x == 2 ? t4.z : t4.w;
+              const float rs = x == 0 ? q4.x : x == 1 ? q4.y : x == 2 ? q4.z : q4.w;
               float v[2];
 #pragma unroll
               for (int j = 0; j < 2; j++) {
                 v[j] = acc[i][j][4 * g + x];
-                if constexpr (Q8) v[j] *= sc[j];
+                if constexpr (Q8) v[j] = (v[j] - 128.f * rs) * sc[j];
                 if (bias) v[j] += bv[j];
                 if (mrw) v[j] *= tw;
               }
