@@ -211,17 +211,20 @@ def fused_moe_down_combine(A, B, B_scale, topk_weights, sorted_ids, experts_ids,
 def fused_moe_gate_up_silu(A, B, B_scale, sorted_ids, experts_ids, ntpp, top_k, block_size,
                            bias=None, out=None, topk_ids_size=None, stream=None):
     """Gate/up expert GEMM with silu_and_mul fused into its epilogue: B int8
-    [E, 2I, K] (gate rows, then up rows) with B_scale [E, 2I], or B in A's
-    dtype (B_scale None) -> [topk_ids_size, I], the same values as
-    invoke_fused_moe followed by silu_and_mul."""
+    [E, 2I, K] (gate rows, then up rows; uint8 is taken as the same bytes) with
+    B_scale [E, 2I], or B in A's dtype (B_scale None) -> [topk_ids_size, I],
+    the same values as invoke_fused_moe followed by silu_and_mul."""
     _need_cuda(A, B, B_scale, sorted_ids, experts_ids, ntpp)
+    q8 = B.dtype in (torch.int8, torch.uint8)
+    if not q8 and B.dtype != A.dtype:
+        raise ValueError(f"experts are int8 or in the activations' dtype: got {B.dtype}, {A.dtype}")
     E, N, K = B.shape
     tis = topk_ids_size if topk_ids_size is not None else A.shape[0] * top_k
     if out is None:
         out = torch.empty(tis, N // 2, dtype=A.dtype, device=A.device)
     tail = (_ptr(bias), _ptr(sorted_ids), _ptr(experts_ids), _ptr(ntpp), A.shape[0], K, N, E, tis,
             top_k, block_size, int(bias is not None), _DT_CODE[A.dtype], stream_ptr(stream))
-    if B.dtype == torch.int8:
+    if q8:
         check(lib.ubridge_fused_moe_w8a16_silu(_ptr(out), _ptr(A), _ptr(B), _ptr(B_scale), *tail))
     else:
         check(lib.ubridge_fused_moe_silu(_ptr(out), _ptr(A), _ptr(B), *tail))
