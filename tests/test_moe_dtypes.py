@@ -56,3 +56,30 @@ def test_gate_up_silu_weight_dtypes(rec, a, b, scales, entry):
     else:
         moe.fused_moe_gate_up_silu(A, B, S, *_routing(), 1, 4)
         assert rec.calls == [entry]
+
+
+@pytest.mark.parametrize("a,b,entry", [
+    (torch.bfloat16, torch.int8, "ubridge_fused_moe_w8a16"),
+    (torch.bfloat16, torch.bfloat16, "invoke_fused_moe_bf16"),
+    (torch.float16, torch.float16, "invoke_fused_moe_f16"),
+    (torch.bfloat16, torch.float16, None), (torch.float16, torch.uint8, None),
+    (torch.bfloat16, torch.float32, None)])
+def test_expert_gemm_weight_dtypes(rec, a, b, entry):
+    A, B, C = torch.zeros(T, K, dtype=a), torch.zeros(E, N, K).to(b), torch.zeros(T, N, dtype=a)
+    S = torch.ones(E, N, dtype=a)
+    call = lambda: moe.invoke_fused_moe(A, B, C, None, *_routing(), 1, 4, False, B_scale=S)
+    if entry is None:
+        with pytest.raises(ValueError):
+            call()
+        assert rec.calls == []
+    else:
+        call()
+        assert rec.calls == [entry]
+    ids = torch.zeros(T, 1, dtype=torch.int32)
+    call = lambda: moe.topsaten_fused_moe_gemm(A, B, None, ids, *_routing(), False, 4)
+    if a == b:
+        call()
+        assert rec.calls[-1] == "topsaten_fused_moe_gemm"
+    else:
+        with pytest.raises(ValueError):
+            call()

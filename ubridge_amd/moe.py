@@ -50,6 +50,13 @@ def device_error(stream=None):
     check(lib.ubridge_device_error(stream_ptr(stream)))
 
 
+def _need_dtype(A, B):
+    """B is read in A's dtype: another one gives wrong numbers, a narrower one
+    is read past its end."""
+    if B.dtype != A.dtype:
+        raise ValueError(f"experts are int8 or in the activations' dtype: got {B.dtype}, {A.dtype}")
+
+
 def topk_softmax(gating, topk, renormalize=True, stream=None):
     """gating [T, E] (f32/f16/bf16) -> (weights [T, topk] same dtype, ids int32)."""
     _need_cuda(gating)
@@ -148,6 +155,7 @@ def topsaten_fused_moe_gemm(A, B, topk_weights, topk_ids, sorted_ids, experts_id
     """The status-returning grouped GEMM (topsaten_moe_wrapper.cpp:152-208):
     A [T, hidden], B [E, inter, hidden] -> C [T, k, inter]."""
     _need_cuda(A, B, sorted_ids, experts_ids, ntpp)
+    _need_dtype(A, B)
     T, hidden = A.shape
     E, inter, _ = B.shape
     k = topk_ids.shape[1]
@@ -167,6 +175,8 @@ def invoke_fused_moe(A, B, C, topk_weights, sorted_ids, experts_ids, ntpp, top_k
     B: [E, N, K] in A's dtype (invoke_fused_moe_*) or int8 with per-channel
     B_scale [E, N] (W8A16).  C: [topk_ids_size, N]."""
     _need_cuda(A, B, C, sorted_ids, experts_ids, ntpp)
+    if B.dtype != torch.int8:
+        _need_dtype(A, B)
     E, N, K = B.shape
     M = A.shape[0]
     tis = topk_ids_size if topk_ids_size is not None else C.shape[0]
@@ -216,8 +226,8 @@ def fused_moe_gate_up_silu(A, B, B_scale, sorted_ids, experts_ids, ntpp, top_k, 
     the same values as invoke_fused_moe followed by silu_and_mul."""
     _need_cuda(A, B, B_scale, sorted_ids, experts_ids, ntpp)
     q8 = B.dtype in (torch.int8, torch.uint8)
-    if not q8 and B.dtype != A.dtype:
-        raise ValueError(f"experts are int8 or in the activations' dtype: got {B.dtype}, {A.dtype}")
+    if not q8:
+        _need_dtype(A, B)
     E, N, K = B.shape
     tis = topk_ids_size if topk_ids_size is not None else A.shape[0] * top_k
     if out is None:
