@@ -50,6 +50,25 @@ def test_quantize_rows_units(dev, dtype, R, C):
     assert np.array_equal(q[~nan], want_q[~nan]) and np.all((q[nan] & 0x7F) == 0x7F)
 
 
+@pytest.mark.parametrize("C", [8, 512])
+def test_quantize_rows_many(dev, C):
+    # more rows than a launch has workgroups of 256 threads (2^32 threads); the
+    # rows with values against the oracle, zero rows: code 0, scale 1
+    R = (1 << 24) + 5
+    x = torch.zeros(R, C, dtype=torch.bfloat16, device=dev)
+    rows = torch.tensor([0, 1, R // 2, (1 << 24) - 1, 1 << 24, R - 1], device=dev)
+    v = torch.randn(rows.numel(), C, generator=torch.Generator().manual_seed(C)).bfloat16()
+    x[rows] = v.to(dev)
+    q, s = fp8.quantize_rows(x)
+    want_q, want_s = oracle.fp8_quantize_rows(v.float().numpy())
+    assert np.array_equal(q[rows].cpu().numpy(), want_q) and np.array_equal(s[rows].cpu().numpy(), want_s)
+    rest = torch.ones(R, dtype=torch.bool, device=dev)
+    rest[rows] = False
+    assert bool((s[rest] == 1.0).all())
+    q[rows] = 0
+    assert not bool(q.any())
+
+
 def test_prepack_transpose(dev):
     w = torch.randint(0, 256, (200, 72), dtype=torch.uint8, device=dev)
     assert torch.equal(fp8.prepack_weight(w), w.T.contiguous())

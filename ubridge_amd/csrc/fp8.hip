@@ -563,6 +563,7 @@ __global__ void __launch_bounds__(NT) k_quant_rows_fp8_v(const uint4* __restrict
 
 template <int DT, int NT>
 bool quant_rows_v(const void* x, uint8_t* q, float* scale, int R, int V, hipStream_t s) {
+  if ((uint64_t)R * NT >= 1ull << 32) return false;  // a launch has fewer than 2^32 threads
   const int nv = ub_cdiv(V, NT);
   const uint4* xv = (const uint4*)x;
   if (nv <= 1) k_quant_rows_fp8_v<DT, NT, 1><<<R, NT, 0, s>>>(xv, q, scale, V);
