@@ -50,6 +50,17 @@ def test_quantize_rows_units(dev, dtype, R, C):
     assert np.array_equal(q[~nan], want_q[~nan]) and np.all((q[nan] & 0x7F) == 0x7F)
 
 
+@pytest.mark.parametrize("R,C", [(1023, 504), (1024, 504), (1024, 512), (4099, 128), (1025, 8)])
+def test_quantize_rows_narrow(dev, R, C):
+    # both sides of the rule for narrow rows (512 values, 1024 rows)
+    x = torch.randn(R, C, generator=torch.Generator().manual_seed(R + C))
+    x[R // 2] = 0.0
+    for t in (torch.float32, torch.bfloat16):
+        q, s = fp8.quantize_rows(x.to(t).to(dev))
+        want_q, want_s = oracle.fp8_quantize_rows(x.to(t).float().numpy())
+        assert np.array_equal(s.cpu().numpy(), want_s) and np.array_equal(q.cpu().numpy(), want_q)
+
+
 @pytest.mark.parametrize("C", [8, 512])
 def test_quantize_rows_many(dev, C):
     # more rows than a launch has workgroups of 256 threads (2^32 threads); the

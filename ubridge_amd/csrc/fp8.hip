@@ -577,10 +577,17 @@ bool quant_rows_v(const void* x, uint8_t* q, float* scale, int R, int V, hipStre
 // Rows of whole 16-byte units (of x; the codes then 8- or 4-byte aligned) up
 // to 8 units per thread take the one-workgroup-per-row form.  256 threads
 // where there are rows for every CU, 1024 below that (and for longer rows).
+// Many rows below 512 values leave most of a workgroup idle and are bound by
+// the rate at which workgroups start, so they take the general form, four rows
+// a workgroup.  bf16, us, general / one workgroup a row: 262144 rows of 64
+// 48.6 / 144, 128 86.5 / 158, 256 148 / 167, 512 277 / 178; 4096 rows of 128
+// 3.9 / 5.2, 256 4.5 / 5.2, 512 5.8 / 5.3; up to 500 rows level at 128, 4.0 /
+// 3.7 at 256.  f32 the same: 262144 rows of 128 88 / 155, 256 156 / 163, 512
+// 285 / 194.
 template <int DT>
 void quant_rows(const void* x, uint8_t* q, float* scale, int R, int C, hipStream_t s) {
   constexpr int E = DT == UB_F32 ? 4 : 8;
-  if (C % E == 0 && ((uintptr_t)x & 15) == 0 && ((uintptr_t)q & (E - 1)) == 0) {
+  if ((C >= 512 || R < 1024) && C % E == 0 && ((uintptr_t)x & 15) == 0 && ((uintptr_t)q & (E - 1)) == 0) {
     const int V = C / E;
     if ((R >= 512 || V <= 256) && quant_rows_v<DT, 256>(x, q, scale, R, V, s)) return;
     if (quant_rows_v<DT, 1024>(x, q, scale, R, V, s)) return;
