@@ -917,7 +917,8 @@ __global__ void __launch_bounds__(256) k_ksum(const float* __restrict__ part, si
 // up to 16 where a part keeps at least 4 units of K-steps (beyond, the longer
 // sum costs what the shorter walk gives: 24 x 4096 x 4096 GPTQ at S = 8 / 16
 // 14.4 / 15.3 us, but 24 x 14336 x 4096 25.7 / 20.7, 64 tokens 28.3 / 25.2,
-// Q4_K 34.5 / 28.4).  S = 1 where the call may not allocate (may_alloc false:
+// Q4_K 34.5 / 28.4).  GGUF weights keep at least one 256-k span a part (Q4_0 512 x
+// 1024 x 1024: 22.0 us as 4 parts, 25.3 as 8).  S = 1 where the call may not allocate (may_alloc false:
 // the allocation-free entry point).  Parts need not be equal: int8 [N, K] 201
 // x 3520 x 9000 (36 tiles of 256 x 256 or 72 of 128 x 256, 55 K-steps) 89 us
 // unsplit, 39 as 72 tiles x 3.
@@ -925,7 +926,7 @@ int pick_ksplit(const W4Args& p, bool split, bool may_alloc) {
   if (!may_alloc || ub_tune(UB_TUNE_W4A16_PATH) == 7) return 1;
   const int units = split ? ub_cdiv(p.K, 128) : p.K / 64;
   const long tiles = (long)ub_cdiv(p.M, split ? (small_tiles(p.M) ? 64 : 128) : 256) * ub_cdiv(p.N, kBN);
-  const int most = std::min(units, std::max(8, std::min(16, units / 4)));
+  const int most = std::min(p.scales ? units : p.K / 256, std::max(8, std::min(16, units / 4)));
   return (int)std::max<long>(1, std::min<long>(most, num_cus() / tiles));
 }
 
