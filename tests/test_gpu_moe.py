@@ -98,6 +98,60 @@ def test_moe_align_many_groups_map_tokens(dev, rt):
     assert np.array_equal(s.cpu().numpy(), os_) and np.array_equal(e.cpu().numpy(), oe)
 
 
+@pytest.mark.parametrize("T,k,E,bs", [(1, 1, 3, 8), (7, 2, 5, 4), (64, 8, 128, 32), (128, 8, 128, 16),
+                                      (129, 8, 128, 32), (341, 3, 1000, 4), (1024, 1, 1024, 32),
+                                      (1024, 1, 1, 64), (1025, 1, 60, 16)])
+def test_moe_align_map_tokens(dev, T, k, E, bs):
+    # expert_map and real_token_num on both sides of the one-workgroup form's
+    # 1024 slots
+    g = np.random.default_rng(T * k + E)
+    ids = g.integers(0, E, (T, k)).astype(np.int32)
+    emap = np.where(np.arange(E) % 3 == 1, -1, np.arange(E) // 2).astype(np.int32)
+    for rt in (None, 0, 1, T // 2, T):
+        for em in (None, emap):
+            s, e, n = moe.moe_align_block_size(
+                torch.from_numpy(ids).to(dev), E, bs, real_token_num=rt,
+                expert_map=None if em is None else torch.from_numpy(em).to(dev))
+            os_, oe, on = oracle.moe_align_block_size(ids, E, bs, real_token_num=rt, expert_map=em)
+            assert n.item() == on[0]
+            assert np.array_equal(s.cpu().numpy(), os_) and np.array_equal(e.cpu().numpy(), oe)
+
+
+@pytest.mark.parametrize("off", [0, 1])  # 16-byte aligned ids or not
+@pytest.mark.parametrize("T", [300, 1701])  # one workgroup; five and the remainder of a 4-id load
+@pytest.mark.parametrize("what", ["neg_first", "big_first", "neg_mid", "big_last", "map", "few", "many"])
+def test_moe_align_refused(dev, off, T, what):
+    # an id, map entry or token count out of range: no blocks, all padding, the
+    # device error set once, nothing written past the outputs
+    k, E, bs = 3, 40, 32
+    ids = np.random.default_rng(T).integers(0, E, T * k).astype(np.int32)
+    emap = np.arange(E, dtype=np.int32)
+    if what == "neg_first":
+        ids[0] = -1
+    elif what == "big_first":
+        ids[1] = E
+    elif what == "neg_mid":
+        ids[T * k // 2] = -7
+    elif what == "big_last":
+        ids[-1] = E + 3
+    elif what == "map":
+        emap[E - 1] = E
+    rt = {"few": -1, "many": T + 1}.get(what, T)
+    buf = torch.zeros(T * k + off, dtype=torch.int32, device=dev)
+    buf[off:] = torch.from_numpy(ids).to(dev)
+    mp = T * k + E * (bs - 1)
+    out = [torch.full((n + 1,), -9, dtype=torch.int32, device=dev) for n in (mp, mp // bs, 1)]
+    em, tn = torch.from_numpy(emap).to(dev), torch.tensor([rt], dtype=torch.int32, device=dev)
+    _lib.lib.moe_align_block_size(*(ops._ptr(o) for o in out), ops._ptr(buf[off:]), ops._ptr(tn),
+                                  ops._ptr(em), E, bs, T, k, ops.stream_ptr())
+    _lib.check()
+    with pytest.raises(_lib.UbridgeError):
+        moe.device_error()
+    moe.device_error()  # cleared
+    assert all(o[-1].item() == -9 for o in out) and out[2][0].item() == 0
+    assert bool((out[0][:-1] == T * k).all()) and not bool(out[1][:-1].any())
+
+
 def test_moe_align_bad_ids_flagged(dev):
     ids = torch.tensor([[0, 1], [2, 9]], dtype=torch.int32, device=dev)
     s, e, n = moe.moe_align_block_size(ids, 4, 2)

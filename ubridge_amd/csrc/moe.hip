@@ -241,8 +241,8 @@ __device__ __forceinline__ uint64_t same_expert(int e, int nbits) {
   return m;
 }
 
-// LDS: before[E], rest[E], eoff[E + 1], cnt[kAlignWaves][E] (16 bits)
-size_t align_lds(int E) { return sizeof(int) * (3 * (size_t)E + 1) + 2 * (size_t)kAlignWaves * E; }
+// LDS: before[E], rest[E], em[E] (the map), eoff[E + 1], cnt[kAlignWaves][E] (16 bits)
+size_t align_lds(int E) { return sizeof(int) * (4 * (size_t)E + 1) + 2 * (size_t)kAlignWaves * E; }
 
 __global__ void __launch_bounds__(kAlignThreads) k_moe_align(
     int* __restrict__ sorted, int* __restrict__ experts, int* __restrict__ ntpp,
@@ -251,7 +251,8 @@ __global__ void __launch_bounds__(kAlignThreads) k_moe_align(
   extern __shared__ int sh[];
   int* before = sh;
   int* rest = before + E;
-  int* eoff = rest + E;
+  int* em = rest + E;
+  int* eoff = em + E;
   uint16_t* cnt = (uint16_t*)(eoff + E + 1);
   __shared__ int bad, wsum[kAlignWaves];
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
@@ -267,8 +268,10 @@ __global__ void __launch_bounds__(kAlignThreads) k_moe_align(
   if (tid == 0) bad = 0;
   for (int i = tid; i < 2 * E; i += kAlignThreads) sh[i] = 0;
   for (int i = tid; i < kAlignWaves * E; i += kAlignThreads) cnt[i] = 0;
-  if (emap)
-    for (int e = tid; e < E; e += kAlignThreads) any_bad |= emap[e] < -1 || emap[e] >= E;
+  for (int e = tid; e < E; e += kAlignThreads) {
+    em[e] = emap ? emap[e] : e;
+    any_bad |= em[e] < -1 || em[e] >= E;
+  }
   __syncthreads();
   auto count = [&](int e, int i) {
     if ((unsigned)e >= (unsigned)E) any_bad = true;
@@ -327,7 +330,7 @@ __global__ void __launch_bounds__(kAlignThreads) k_moe_align(
       const int mid = (lo + hi) >> 1;
       if (eoff[mid] <= v) lo = mid; else hi = mid;
     }
-    experts[b] = v >= total ? 0 : emap ? emap[lo] : lo;
+    experts[b] = v >= total ? 0 : em[lo];
   }
   if (g == 0 && tid == 0) {
     ntpp[0] = total;
@@ -360,10 +363,9 @@ __global__ void __launch_bounds__(kAlignThreads) k_moe_align(
 }
 
 // ======================================== moe_align for small slot counts
-// The same outputs as k_moe_align (no expert_map / real_token_num), for
-// n = T*k <= 1024 slots in one workgroup of 1024 threads (8 / 256 / 1024 slots
-// of 128 experts 4.8 / 5.0 / 6.0 us, k_moe_align 5.8 / 5.9 / 6.4; at 2048 7.0
-// and 6.1).  Slots are cut
+// The same outputs as k_moe_align for T*k <= 1024 slots in one workgroup of
+// 1024 threads (8 / 256 / 1024 slots of 128 experts 4.8 / 5.0 / 6.0 us,
+// k_moe_align 5.8 / 5.9 / 6.4; at 2048 7.0 and 6.1).  Slots are cut
 // into chunks of 64, one wavefront-wide chunk per (wave, q).  Within a chunk
 // the lanes holding the same expert are found by one ballot per bit of the
 // expert id (log2 E ballots), so a slot's rank among equal experts before it
@@ -377,25 +379,33 @@ constexpr int kRouteThreads = 1024, kRouteWaves = kRouteThreads / 64, kRouteMaxN
 constexpr int kRouteQ = kRouteMaxN / 64 / kRouteWaves;  // chunks per wave
 
 // The align, by the whole 1024-thread workgroup; ids in global memory or
-// LDS, sh the LDS scratch sized by align_small_lds.
+// LDS, sh the LDS scratch sized by align_small_lds for T*k slots.
 __device__ __forceinline__ void align_small_body(const int* ids, int* sh, int* sorted, int* experts,
-                                                 int* ntpp, int n, int E, int bs) {
-  const int nc = (n + 63) / 64;
+                                                 int* ntpp, const int* real_tn, const int* emap,
+                                                 int E, int bs, int T, int k) {
+  int tn = real_tn ? *real_tn : T;
+  bool any_bad = tn < 0 || tn > T;
+  if (any_bad) tn = 0;
+  const int n = tn * k, pad = T * k, nc = (pad + 63) / 64;
   // chunk groups for the prefix over chunks: G groups of CPG chunks per expert
   const int G = max(1, min(nc, kRouteThreads / E)), CPG = (nc + G - 1) / G;
   int* cnt = sh;             // [nc][E]: counts, then exclusive prefix over chunks
   int* part = cnt + nc * E;  // [G][E]: per-group sums, then their exclusive prefix
   int* eoff = part + G * E;  // [E + 1] padded expert offsets
-  int& bad = eoff[E + 1];
+  int* em = eoff + E + 1;    // [E] the map (a load here, not in the chain of the last step)
+  int& bad = em[E];
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  const int pad = n, max_padded = n + E * (bs - 1), max_blocks = max_padded / bs;
+  const int max_padded = pad + E * (bs - 1), max_blocks = max_padded / bs;
   const int nbits = E > 1 ? 32 - __clz(E - 1) : 0;
   if (tid == 0) bad = 0;
   for (int i = tid; i < nc * E; i += kRouteThreads) cnt[i] = 0;
   for (int i = tid; i < max_padded; i += kRouteThreads) sorted[i] = pad;
   for (int i = tid; i < max_blocks; i += kRouteThreads) experts[i] = 0;
+  for (int e = tid; e < E; e += kRouteThreads) {
+    em[e] = emap ? emap[e] : e;
+    any_bad |= em[e] < -1 || em[e] >= E;
+  }
   int ex[kRouteQ];
-  bool any_bad = false;
 #pragma unroll
   for (int q = 0; q < kRouteQ; q++) {
     const int i = (wv + q * kRouteWaves) * 64 + lane;
@@ -479,22 +489,23 @@ __device__ __forceinline__ void align_small_body(const int* ids, int* sh, int* s
       const int mid = (lo + hi) >> 1;
       if (eoff[mid] <= v) lo = mid; else hi = mid;
     }
-    experts[b] = lo;
+    experts[b] = em[lo];
   }
   if (tid == 0) ntpp[0] = total;
 }
 
 __global__ void __launch_bounds__(kRouteThreads) k_moe_align_small(
     const int* __restrict__ ids, int* __restrict__ sorted, int* __restrict__ experts,
-    int* __restrict__ ntpp, int n, int E, int bs) {
+    int* __restrict__ ntpp, const int* __restrict__ real_tn, const int* __restrict__ emap, int E,
+    int bs, int T, int k) {
   extern __shared__ int sh[];
-  align_small_body(ids, sh, sorted, experts, ntpp, n, E, bs);
+  align_small_body(ids, sh, sorted, experts, ntpp, real_tn, emap, E, bs, T, k);
 }
 
 size_t align_small_lds(int n, int E) {
   const int nc = (n + 63) / 64;
   const int G = std::max(1, std::min(nc, kRouteThreads / E));
-  return sizeof(int) * ((size_t)nc * E + (size_t)G * E + E + 2);
+  return sizeof(int) * ((size_t)nc * E + (size_t)G * E + 2 * E + 2);
 }
 
 // Top-k and align of at most kRouteTokens tokens in one workgroup, a wavefront
@@ -510,16 +521,16 @@ __global__ void __launch_bounds__(kRouteThreads) k_moe_route_small(
   topk_tokens<DT, G, NPL>(in, out, ids, wf32, nullptr, threadIdx.x / G, kRouteThreads / G, T, E, k,
                           norm, threadIdx.x % G);
   __syncthreads();
-  align_small_body(ids, sh, sorted, experts, ntpp, T * k, E, bs);
+  align_small_body(ids, sh, sorted, experts, ntpp, nullptr, nullptr, E, bs, T, k);
 }
 
 bool align_small_ok(int n, int E) { return n > 0 && n <= kRouteMaxN && align_small_lds(n, E) <= 96 * 1024; }
-void align_small_launch(const int* ids, int* sorted, int* experts, int* ntpp, int n, int E, int bs,
-                        hipStream_t s) {
-  const size_t lds = align_small_lds(n, E);
+void align_small_launch(const int* ids, int* sorted, int* experts, int* ntpp, const int* real_tn,
+                        const int* emap, int E, int bs, int T, int k, hipStream_t s) {
+  const size_t lds = align_small_lds(T * k, E);
   (void)hipFuncSetAttribute((const void*)k_moe_align_small, hipFuncAttributeMaxDynamicSharedMemorySize,
                       (int)lds);
-  k_moe_align_small<<<1, kRouteThreads, lds, s>>>(ids, sorted, experts, ntpp, n, E, bs);
+  k_moe_align_small<<<1, kRouteThreads, lds, s>>>(ids, sorted, experts, ntpp, real_tn, emap, E, bs, T, k);
 }
 
 // ======================================================== grouped expert GEMM
@@ -1110,9 +1121,9 @@ static int moe_align_launch(int* sorted_ids, int* experts_ids, int* num_tokens_p
              block_size, token_num, topk);
   UB_REQUIRE(sorted_ids && experts_ids && num_tokens_post_pad && (topk_ids || token_num == 0),
              "%s: null pointer", nm);
-  if (!real_token_num && !expert_map && align_small_ok(token_num * topk, num_experts)) {
-    align_small_launch(topk_ids, sorted_ids, experts_ids, num_tokens_post_pad, token_num * topk,
-                       num_experts, block_size, ub_stream(stream));
+  if (align_small_ok(token_num * topk, num_experts)) {
+    align_small_launch(topk_ids, sorted_ids, experts_ids, num_tokens_post_pad, real_token_num,
+                       expert_map, num_experts, block_size, token_num, topk, ub_stream(stream));
     return ub_check_launch(nm);
   }
   // one wavefront-wide chunk per wavefront and workgroup, up to a workgroup per CU
