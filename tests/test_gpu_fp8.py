@@ -85,12 +85,15 @@ def test_prepack_transpose(dev):
     assert torch.equal(fp8.prepack_weight(w), w.T.contiguous())
 
 
-@pytest.fixture(params=[0, 3, 2, 4], ids=["default", "own_bk128", "4_waves", "8_waves_bk64"])
+@pytest.fixture(params=[0, 1, 3, 2, 4],
+                ids=["default", "hipblaslt", "own_bk128", "4_waves", "8_waves_bk64"])
 def fp8_variant(request):
-    # gemm_tile knob: 0 the default (hipBLASLt's fp8 GEMM with row / column
-    # scale vectors where it serves the shape, else the kernel of 3), 3 the
-    # library's own kernel (128-byte K-steps when K % 128 == 0, else 64-byte
-    # ones), 2 its 4-wavefront kernel, 4 the 8-wavefront 64-byte one
+    # gemm_tile knob: 0 the default (up to 16 tokens the decode kernel, for K a
+    # multiple of 128 up to 8192; else hipBLASLt's fp8 GEMM with row / column
+    # scale vectors where it serves the shape, else the kernel of 3), 1 that
+    # without the decode kernel, 3 the library's own kernel (128-byte K-steps
+    # when K % 128 == 0, else 64-byte ones), 2 its 4-wavefront kernel, 4 the
+    # 8-wavefront 64-byte one
     ops.tune_set("gemm_tile", request.param)
     yield request.param
     ops.tune_set("gemm_tile", 0)
@@ -116,11 +119,28 @@ def test_fp8_gemm_vs_oracle(dev, fp8_variant, M, K, N):
 
 
 @pytest.mark.parametrize("K,N", [(128, 8), (384, 40), (1024, 16400), (1152, 520), (1920, 8200),
-                                 (2176, 4099), (4096, 16400), (4224, 300), (8192, 4136)])
+                                 (1152, 16400), (2048, 28688), (2176, 4099), (4096, 16400), (4224, 300),
+                                 (8192, 4136)])
 @pytest.mark.parametrize("M", [1, 7, 16])
 def test_fp8_decode(dev, M, K, N):
     # up to 16 tokens: every step count / tile width of the decode kernel, K
     # with idle wavefronts, ragged N, more than one tile per workgroup
+    _few_tokens(dev, M, K, N)
+
+
+@pytest.mark.parametrize("knob,M,K,N", [(0, 16, 8320, 200), (0, 3, 14336, 264), (0, 5, 192, 72),
+                                        (0, 16, 1088, 520), (1, 1, 128, 40), (1, 16, 4096, 264)])
+def test_fp8_few_tokens_gemm(dev, knob, M, K, N):
+    # up to 16 tokens outside the decode kernel's contract (K > 8192, K % 128)
+    # or with the knob that leaves it out: the GEMM
+    ops.tune_set("gemm_tile", knob)
+    try:
+        _few_tokens(dev, M, K, N)
+    finally:
+        ops.tune_set("gemm_tile", 0)
+
+
+def _few_tokens(dev, M, K, N):
     g = torch.Generator(device=dev).manual_seed(M + K + N)
     aq, sa = fp8.quantize_rows(torch.randn(M, K, device=dev, generator=g))
     wq, sw = fp8.quantize_rows(torch.randn(N, K, device=dev, generator=g))
