@@ -2160,11 +2160,12 @@ struct MmCfg {
 // for the first (each lane's 16 k lie in one block, so a lane reads either
 // its token's row or the zero row of an unused slot), and the two slots' sums
 // are added at the end.  Same products, half the scaling, 16-byte instead of
-// 8-byte LDS reads.  Quantize + GEMV at 8 tokens in a graph, weights from HBM
-// (us, before / after; K x N): Q8_0 4096 x 28672 29.2 / 27.7, 4096 x 6144 12.2
-// / 11.8, 4096 x 4096 10.4 / 10.0, 14336 x 4096 18.6 / 18.1; Q4_0 21.2 / 17.8,
-// 10.5 / 9.2, 8.6 / 8.0, 15.1 / 13.9; Q4_K 19.2 / 18.5, 9.9 / 9.7, 9.1 / 9.0,
-// 15.2 / 15.1.  5 to 7 tokens: as 8.
+// 8-byte LDS reads.  Quantize + GEMV at 8 tokens in a graph, weights from HBM,
+// the two in turn in one run (us, one block / two blocks a product; K x N): Q8_0
+// 4096 x 28672 28.5 / 26.9, 4096 x 6144 12.6 / 12.0, 4096 x 4096 10.6 / 10.2,
+// 14336 x 4096 19.3 / 18.7; Q4_0 21.8 / 18.5, 10.4 / 9.2, 8.6 / 8.1, 15.2 / 14.1;
+// Q4_K (whose scaling is integer: 1 to 2%) 19.6 / 19.1, 9.9 / 9.8, 9.2 / 9.1,
+// 15.5 / 15.4.  5 tokens: the same ratios, Q4_K 14336 x 4096 14.9 / 15.0.
 template <int QT, int OT, int RWV, int KG, int SB, int D, int HK, bool T8>
 __global__ void __launch_bounds__(64 * RWV * KG) k_gemv_mm(GemvArgs a) {
   using C = MmCfg<QT, RWV, KG, SB>;
@@ -2554,8 +2555,8 @@ template <int QT, int OT>
 void launch_mm(int cfg, const GemvArgs& a, hipStream_t s) {
   if (cfg <= 0) {
     cfg = a.N >= 16384 ? (QT == UB_Q8_0 ? 1 : 13) : a.N > 4096 ? 5 : 7;
-    if (a.M <= 8) {  // the same shapes, two blocks per product (faster at every
-                     // size and format measured, see k_gemv_mm)
+    if (a.M <= 8) {  // the same shapes, two blocks per product: 3 to 16% faster
+                     // for Q8_0 / Q4_0, 0 to 3% for Q4_K (see k_gemv_mm)
       if (cfg == 1) return launch_mm_t<QT, OT, 7, 1, 1, 3, 16, true>(a, s);
       if (cfg == 13) return launch_mm_t<QT, OT, 7, 2, 1, 2, 16, true>(a, s);
       if (cfg == 5) return launch_mm_t<QT, OT, 2, 4, 1, 2, 56, true>(a, s);

@@ -84,8 +84,7 @@ k_moe_tile(MoeArgs a, int* err) {
   constexpr int WB = Q8 ? 1 : 2;
   constexpr int RA = BK * 2, UA = RA / 16;    // A row bytes / 16-byte units
   constexpr int RB = BK * WB, UB = RB / 16;   // weight row bytes / units
-  constexpr int AR = kTM * RA < 1024 * NWV ? 1024 * NWV / RA : kTM;  // A rows in LDS: a load per wave
-  constexpr int AB = AR * RA, BB = BN * RB, STB = AB + BB;
+  constexpr int AB = kTM * RA, BB = BN * RB, STB = AB + BB;
   constexpr int NA = AB / 1024 / NWV, NB = BB / 1024 / NWV, NL = NA + NB;  // loads per wave, stage
   static_assert(kTM == 128 || kTM == 64 || kTM == 32, "rows of a tile");
   static_assert(AB % (1024 * NWV) == 0 && BB % (1024 * NWV) == 0, "loads split evenly");
@@ -208,7 +207,7 @@ k_moe_tile(MoeArgs a, int* err) {
 #pragma unroll
     for (int j = 0; j < NA; j++) {
       const int u = (j * NWV + wave) * 64 + lane, r = u / UA, c = (u % UA) ^ swa(r);
-      const int s = AR == kTM || r < kTM ? srow[buf][r % kTM] : -1;
+      const int s = srow[buf][r];
       voA[j] = s >= 0 ? (uint32_t)(((size_t)(s / a.a_div) * K + 8 * c) * 2) : kDmaOOB;
     }
 #pragma unroll
@@ -472,17 +471,26 @@ void launch(const MoeArgs& a, int* err, hipStream_t s) {
 // expert).  Whole layers of 128 / 64 / 8 experts (top-8 2048 -> 2 x 768, top-6
 // 2048 -> 2 x 1408, top-2 4096 -> 2 x 1024), us:
 //  * taller tiles need rows to fill them.  int8, 128 experts, k_moe_gemm / 32 /
-//    64 / 128 rows at r = 2: 121 / 125 / - / 147, 4: 137 / 132 / 135 / 164, 16:
-//    163 / 163 / 169 / 181, 24: 180 / 170 / 172 / 184, 48: 243 / 218 / 199 /
-//    220, 96: 379 / - / 267 / 263, 128: 475 / - / 327 / 303; 64 experts at r =
-//    3: 121 / 119 / 121 / 146, 24: 163 / 153 / 151 / 179.  16-bit (no widening
-//    to share) k_moe_gemm / 64 / 128 rows at r = 4: 253 / 250 / 250, 8: 263 /
-//    261 / 261, 24: 286 / 280 / 279, 64: 404 / 336 / 348, 80: 467 / 389 / 347.
+//    64 / 128 rows in turn in one run at r = 2: 123 / 128 / 130 / 147, 3: 133 /
+//    131 / 134 / 151, 8: 147 / 141 / 143 / 160, 16: 163 / 165 / 159 / 171, 24:
+//    178 / 167 / 173 / 176, 32: 195 / 183 / 185 / 186, 48: 229 / 217 / 190 / 210,
+//    64: 267 / 267 / 218 / 229, 96: 351 / 338 / 263 / 246, 128: 441 / 439 / 323 /
+//    284; 64 experts at r = 3: 124 / 121 / 123 / 139, 12: 138 / 132 / 133 / 147,
+//    24: 160 / 156 / 147 / 156, 48: 212 / 202 / 179 / 182: within 5% of the best
+//    up to 64 rows and 7% at 96, as the tiles come out.  16-bit (no widening to
+//    share) k_moe_gemm / 64 / 128 rows, 128 experts at r = 4: 247 / 247 / 252, 8:
+//    264 / 266 / 273, 16: 279 / 275 / 282, 24: 286 / 301 / 290, 38: 320 / 312 /
+//    316, 50: 360 / 327 / 339, 63: 400 / 341 / 350; the two GEMMs alone (64 / 128)
+//    at r = 75: 331 / 326, 94: 380 / 344, 150: 487 / 417; 64 experts at r = 14: 235 /
+//    239, 28: 260 / 246, 47: 283 / 263, 94: 359 / 316: 64 rows are up to 3% faster
+//    below 64 rows of 128 experts, 128 rows up to 20% beyond and for 64 experts.
 //  * at least 160 pairs (128 int8 rows: 512): each walks all of K, so few of
-//    them leave the chip idle.  8 experts, int8 gate/up, k_moe_gemm / 32 / 64 /
-//    128 rows at r = 32 (96 / 64 / 64 pairs) 35 / 41 / 49 / 64, 64 (160 / 96 /
-//    64) 44 / 41 / 50 / 73, 128 (- / 160 / 96) 60 / 57 / 51 / 73, 256 (- / 288 /
-//    160) 100 / 85 / 70 / 78.
+//    them leave the chip idle.  8 experts, int8 layer, k_moe_gemm / 32 / 64 / 128
+//    rows at r = 32 (gate/up 96 / 64 / 64 pairs) 64 / 71 / 81 / 99, 64 (160 / 96 /
+//    64) 84 / 78 / 83 / 111, 128 (- / 160 / 96) 121 / 104 / 92 / 117, 256 (- / 288 /
+//    160) 184 / 148 / 129 / 133.  16-bit calls with too few pairs of 128 rows take
+//    64: 8 experts at r = 175 (gate/up 119 / 206 pairs), the two GEMMs with 128 / 64
+//    rows, 121 / 108.
 int ub_moe_tile_rows(const MoeArgs& a, bool q8) {
   const long cols = ub_cdiv(a.act ? a.N / 2 : a.N, a.act ? kCols / 2 : kCols);
   auto pays = [&](int rows, int r, long pairs) {
