@@ -566,7 +566,7 @@ def test_pipelined_k_split_over_workgroups(dev, M):
 
 @pytest.mark.parametrize("bits,rhs_t", [(4, 0), (8, 0), (8, 1)])
 @pytest.mark.parametrize("M,K,N", [(40, 192, 264), (130, 192, 64), (33, 704, 1000), (150, 3520, 520),
-                                   (64, 8256, 72), (300, 960, 776)])
+                                   (64, 8256, 72), (300, 960, 776), (40, 1408, 264), (90, 1088, 520)])
 def test_pipelined_uneven_k_split(dev, bits, rhs_t, M, K, N):
     # odd numbers of 64-k steps (the upper K-half then has one step past K) and
     # parts of different lengths, against f64; a row of NaN and one of

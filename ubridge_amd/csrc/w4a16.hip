@@ -912,22 +912,35 @@ __global__ void __launch_bounds__(256) k_ksum(const float* __restrict__ part, si
 
 // Split over K across workgroups for grids that leave CUs idle: with fewer
 // tiles than half the CUs, each tile's K-steps are cut in S nearly equal
-// parts, as many as the CUs take (tiles x S <= CUs); the parts' f32 sums go to
-// the stream's workspace and k_ksum adds them in a fixed order.  S up to 8, and
-// up to 16 where a part keeps at least 4 units of K-steps (beyond, the longer
-// sum costs what the shorter walk gives: 24 x 4096 x 4096 GPTQ at S = 8 / 16
-// 14.4 / 15.3 us, but 24 x 14336 x 4096 25.7 / 20.7, 64 tokens 28.3 / 25.2,
-// Q4_K 34.5 / 28.4).  GGUF weights keep at least one 256-k span a part (Q4_0 512 x
-// 1024 x 1024: 22.0 us as 4 parts, 25.3 as 8).  S = 1 where the call may not allocate (may_alloc false:
-// the allocation-free entry point).  Parts need not be equal: int8 [N, K] 201
-// x 3520 x 9000 (36 tiles of 256 x 256 or 72 of 128 x 256, 55 K-steps) 89 us
-// unsplit, 39 as 72 tiles x 3.
+// parts (tiles x S <= CUs); the parts' f32 sums go to the stream's workspace and
+// k_ksum adds them in a fixed order.  S is where the longest part's walk (1 us per
+// unit of K-steps, 0.8 us on 64-row tiles) and the sum (2 us, and 0.1 us + 0.45 us
+// per million outputs for each part) are together shortest, so also the fewest
+// parts with that longest one; up to 8, up to 16 where a part keeps at least 4
+// units, and GGUF weights at least a 256-k span.  Fitted to 2390 calls (GPTQ,
+// uint8 4-bit, int8 in both layouts, Q4_K, Q8_0; K 1024 to 14336, N 512 to 28672,
+// 17 to 900 tokens, each at every S): 0.6% over the best of them on average, as many
+// parts as the CUs take 1.7%, a power of two that divides K 7.6%.  us at S: GPTQ
+// 900 x 1024 x 512 1: 23.3, 4: 20.4, 8: 23.4; int8 64 x 1536 x 6144 1: 21.8, 4:
+// 16.8, 8: 19.2; Q8_0 512 x 2048 x 8192 1: 43.9, 2: 38.8; GPTQ 33 x 14336 x 2048 8:
+// 26.3, 16: 19.5; int8 201 x 3520 x 9000 (36 tiles of 256 x 256 or 72 of 128 x 256,
+// 55 K-steps) 89 unsplit, 39 as 72 tiles x 3.  S = 1 where the call may not allocate
+// (may_alloc false: the allocation-free entry point).
 int pick_ksplit(const W4Args& p, bool split, bool may_alloc) {
   if (!may_alloc || ub_tune(UB_TUNE_W4A16_PATH) == 7) return 1;
+  const bool low = split && small_tiles(p.M);  // 64-row tiles
   const int units = split ? ub_cdiv(p.K, 128) : p.K / 64;
-  const long tiles = (long)ub_cdiv(p.M, split ? (small_tiles(p.M) ? 64 : 128) : 256) * ub_cdiv(p.N, kBN);
-  const int most = std::min(p.scales ? units : p.K / 256, std::max(8, std::min(16, units / 4)));
-  return (int)std::max<long>(1, std::min<long>(most, num_cus() / tiles));
+  const long tiles = (long)ub_cdiv(p.M, split ? (low ? 64 : 128) : 256) * ub_cdiv(p.N, kBN);
+  const long most = std::min<long>(num_cus() / tiles, std::min(p.scales ? units : p.K / 256,
+                                                               std::max(8, std::min(16, units / 4))));
+  const double unit = low ? 0.8 : 1.0, part = 0.1 + 0.45e-6 * p.M * p.N;
+  int S = 1;
+  double best = unit * units;
+  for (int s = 2; s <= most; s++) {
+    const double us = unit * ub_cdiv(units, s) + 2.0 + part * s;
+    if (us < best) best = us, S = s;
+  }
+  return S;
 }
 
 // Scratch for the K split picked above (none when S == 1); sets p.ksplit and
